@@ -18,7 +18,7 @@ import torch
 
 from tuvok_amd import (DISPATCH_GROUPS, DISPATCH_QUEUES, GEN_BLOBS, GEN_ELLIPSOID_SDF, GEN_FBM_SHELLS, GEN_PHANTOM,
                        RM_1DTRANS, RM_2DTRANS, RM_ISOSURFACE, HIPRaycaster, RenderBatch, _abi)
-from tuvok_amd.stepnet import StepNet, train_proposal
+from tuvok_amd.stepnet import StepNet, labels, split_samples
 
 ERT = 2.0 ** -11
 GENERATORS = {"blobs": GEN_BLOBS, "fbm": GEN_FBM_SHELLS, "sdf": GEN_ELLIPSOID_SDF, "phantom": GEN_PHANTOM}
@@ -189,6 +189,17 @@ def _look(ren, case, seed, eye=2.0):
     ren.Resize(case["w"], case["h"])
 
 
+def _proposal(ren, rots, seed):
+    """A step network trained on recorded chunks of these views, always in the same order."""
+    rec = ren.GenerateSegments(rots, 50000, seed=seed, fit=True)[:, :42]
+    rec = np.ascontiguousarray(rec)
+    rec = rec[np.argsort(rec.view("V168").reshape(-1), kind="stable")]
+    net = StepNet(0, seed=seed)
+    net.set_data(split_samples(rec)[0], labels(rec, 0.25 / 255, 0.125 / 255))
+    net.train(epochs=4, seed=seed)
+    return net
+
+
 class _DeviceFrames:
     """Frames that a renderer left on the device, for torch to wrap without a copy: the tensor holds this object, and
     with it the renderer that owns the memory."""
@@ -221,7 +232,7 @@ def prepare(case, seed):
         net = None
         if case["step"] == "learned":
             ren.Resize(240, 135)
-            net, _ = train_proposal(ren, [_rotation(a) for a in _angles(seed + 1, 4)], cap=50000, epochs=4, seed=seed)
+            net = _proposal(ren, [_rotation(a) for a in _angles(seed + 1, 4)], seed)
             ren.Resize(case["w"], case["h"])
             ren.SetStepProposal(net, margin=1.0, skip_threshold=0.999, fallback_bound=0.01)
         if case["gen"] in ("phantom", "sdf"):
