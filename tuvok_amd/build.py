@@ -19,7 +19,9 @@ ARCH = os.environ.get("TVK_OFFLOAD_ARCH", "gfx950")
 # (source, extra flags).  The march kernel must not contract a*b+c into FMAs:
 # its float operations mirror the host planner's and the reference restatement's.
 SOURCES = [
-    ("kernels/march.hip", ["-ffp-contract=off"]),
+    ("kernels/march.hip", ["-ffp-contract=off", "-DTVK_MARCH_MODE=0"]),   # once per render mode
+    ("kernels/march.hip", ["-ffp-contract=off", "-DTVK_MARCH_MODE=1"]),
+    ("kernels/march.hip", ["-ffp-contract=off", "-DTVK_MARCH_MODE=2"]),
     ("kernels/bricking.hip", []),
     ("kernels/generate.hip", []),
     ("kernels/stepnet.hip", []),
@@ -48,7 +50,8 @@ COMMON = [
 def _compile(item):
     src, extra = item
     path = os.path.join(CSRC, src)
-    obj = os.path.join(BUILD, src.replace("/", "_") + ".o")
+    mode = "".join(f[-1] for f in extra if f.startswith("-DTVK_MARCH_MODE="))
+    obj = os.path.join(BUILD, src.replace("/", "_") + mode + ".o")
     cmd = [HIPCC, "-c", path, "-o", obj] + COMMON + extra
     if src.endswith(".cpp"):
         cmd = [HIPCC, "-x", "hip", "-c", path, "-o", obj] + COMMON + extra

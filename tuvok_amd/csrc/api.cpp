@@ -1422,9 +1422,9 @@ int render_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_
         a.xcd_count[x] = std::min(per, groups - a.xcd_start[x]);
       }
     }
-    rc = ensure(c, &c->d_queues, &c->queues_cap, 8);
+    rc = ensure(c, &c->d_queues, &c->queues_cap, QUEUE_WORDS);
     if (rc) return rc;
-    HIPCHK(c, launch_fill_u32(c->d_queues, 8u, 0u, c->stream));
+    HIPCHK(c, launch_fill_u32(c->d_queues, QUEUE_WORDS, 0u, c->stream));
     a.queues = c->d_queues;
   }
   if (c->count) HIPCHK(c, hipMemsetAsync(c->d_counter, 0, sizeof(unsigned long long), c->stream));

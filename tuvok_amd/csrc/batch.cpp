@@ -246,6 +246,7 @@ int plan_batch(tvk_batch* b, uint32_t* bricks_total) {
     a.touched = b->count ? b->d_touched : nullptr;
     a.nreq = (int)(k - first);
     a.tiles_total = tiles;
+    chunk_items(tiles, a.xcd_items);
     a.tile_w = tw;
     a.tile_h = th;
     int per_cu = b->tune.groups_per_cu;
@@ -253,7 +254,8 @@ int plan_batch(tvk_batch* b, uint32_t* bricks_total) {
       hipError_t e = (hipError_t)batch_occupancy(L.mode, L.lit, L.bpv, b->count, L.learn, &per_cu);
       if (e != hipSuccess || per_cu <= 0) per_cu = 2;
     }
-    L.groups = ((b->cu_count * per_cu) + 7) & ~7;
+    // a workgroup takes four tiles at once: no more of them than the tiles keep busy
+    L.groups = std::min(((b->cu_count * per_cu) + 7) & ~7, (int)((a.xcd_items[0] + 3u) / 4u) * 8);
     b->launches.push_back(L);
   }
   *bricks_total = (uint32_t)nlist;
@@ -309,7 +311,7 @@ int tvk_batch_create(tvk_batch** out, int device) {
   tvk_default_tuning(&b->tune);
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_queues, 8 * sizeof(unsigned int));
+  if (e == hipSuccess) e = hipMalloc((void**)&b->d_queues, QUEUE_WORDS * sizeof(unsigned int));
   if (e == hipSuccess) e = hipMalloc((void**)&b->d_counter, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipEventCreate(&b->ev[0]);
   if (e == hipSuccess) e = hipEventCreate(&b->ev[1]);

@@ -150,7 +150,7 @@ struct tvk_ctx {
   size_t views_cap = 0;
   uint32_t* d_order = nullptr;   // dispatch order of the 16x16 groups
   size_t order_cap = 0;
-  unsigned int* d_queues = nullptr;   // the persistent launch's 8 XCD work queues
+  unsigned int* d_queues = nullptr;   // the persistent launches' XCD work queues (QUEUE_WORDS)
   size_t queues_cap = 0;
   float* d_out = nullptr;
   size_t out_cap = 0;

@@ -109,18 +109,26 @@ typedef uint32_t tvk_u32x3_a4 __attribute__((ext_vector_type(3), aligned(4)));
 typedef uint32_t tvk_u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t tvk_u32_a1 __attribute__((aligned(1)));
 typedef uint16_t tvk_u16_a1 __attribute__((aligned(1)));
+template <typename T> struct Run4 { typedef tvk_u32x2_a4 Word; };
+template <> struct Run4<uint16_t> { typedef tvk_u32x3_a4 Word; };
 template <typename T>
-__device__ __forceinline__ void run4(const uint8_t* __restrict__ b, uint32_t r, int s, uint32_t o[4]) {
-  if (sizeof(T) == 2) {
-    const tvk_u32x3_a4 w = *reinterpret_cast<const tvk_u32x3_a4*>(b + (r + 4u * (uint32_t)(s >> 1)));
+__device__ __forceinline__ typename Run4<T>::Word run4_load(const uint8_t* __restrict__ b, uint32_t r, int s) {
+  return *reinterpret_cast<const typename Run4<T>::Word*>(b + (r + 4u * (uint32_t)(s >> (sizeof(T) == 2 ? 1 : 2))));
+}
+template <typename T>
+__device__ __forceinline__ void run4_take(typename Run4<T>::Word w, int s, uint32_t o[4]) {
+  if constexpr (sizeof(T) == 2) {
     const uint32_t sh = (uint32_t)(s & 1) * 2u;
     const uint32_t lo = __builtin_amdgcn_alignbyte(w.y, w.x, sh), hi = __builtin_amdgcn_alignbyte(w.z, w.y, sh);
     o[0] = lo & 0xffffu; o[1] = lo >> 16; o[2] = hi & 0xffffu; o[3] = hi >> 16;
   } else {
-    const tvk_u32x2_a4 w = *reinterpret_cast<const tvk_u32x2_a4*>(b + (r + 4u * (uint32_t)(s >> 2)));
     const uint32_t v = __builtin_amdgcn_alignbyte(w.y, w.x, (uint32_t)(s & 3));
     o[0] = v & 0xffu; o[1] = (v >> 8) & 0xffu; o[2] = (v >> 16) & 0xffu; o[3] = v >> 24;
   }
+}
+template <typename T>
+__device__ __forceinline__ void run4(const uint8_t* __restrict__ b, uint32_t r, int s, uint32_t o[4]) {
+  run4_take<T>(run4_load<T>(b, r, s), s, o);
 }
 template <typename T>
 __device__ __forceinline__ void run2(const uint8_t* __restrict__ b, uint32_t r, uint32_t o[2]) {
@@ -130,6 +138,47 @@ __device__ __forceinline__ void run2(const uint8_t* __restrict__ b, uint32_t r, 
   } else {
     const uint32_t w = *reinterpret_cast<const tvk_u16_a1*>(b + r);
     o[0] = w & 0xffu; o[1] = w >> 8;
+  }
+}
+
+// Work distribution of the persistent launches (256-thread workgroups, a grid
+// that is a multiple of 8 so that every queue has waves of its own): XCD x has
+// items[x] tiles; work(x, t) renders tile t of XCD x with one wave.  A queue with
+// no more tiles than its XCD has waves needs no counter: every wave takes the
+// tile of its own number.  From a longer one every tile is drawn with an atomic
+// (a first tile by number measured slower there: 5.65 against 4.83 ms for a
+// 1080p isosurface frame, most costly groups first).  Once its queue is drained
+// a wave reads the 8 counters with one load and draws from the queues that still
+// have tiles, the nearest first; when none has, it exits.  Counters only grow,
+// and a queue's own waves leave it only when its counter says it is empty, so
+// every tile is taken once.  Before, every wave found the 8 queues empty with 8
+// atomics of its own on one cache line: 1024 workgroups took 0.5 ms for that,
+// whatever the frame (64x64 frame of 64^3: 572 us of kernel, now 0.2 ms).
+template <typename F>
+__device__ __forceinline__ void pull_tiles(unsigned int* __restrict__ queues, const uint32_t* items, F&& work) {
+  const uint32_t lane = threadIdx.x & 63u, xcd = blockIdx.x & 7u;
+  const uint32_t waves = (gridDim.x >> 3) * 4u;   // of each XCD
+  uint32_t x = xcd;
+  uint32_t own = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x >> 3) * 4u + (threadIdx.x >> 6)));
+  for (;;) {
+    uint32_t t = own;
+    own = 0xffffffffu;
+    if (waves < items[x]) {
+      if (lane == 0u) t = atomicAdd(queues + x * QUEUE_STRIDE, 1u);
+      t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+    }
+    if (t >= items[x]) {
+      // this queue is drained: the others' counters, one per lane
+      const uint32_t y = (xcd + lane) & 7u;
+      bool left = false;
+      if (lane < 8u && waves < items[y])
+        left = __hip_atomic_load(queues + y * QUEUE_STRIDE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < items[y];
+      const uint64_t m = __ballot(left);
+      if (m == 0) return;
+      x = (xcd + (uint32_t)__ffsll((unsigned long long)m) - 1u) & 7u;
+      continue;
+    }
+    work(x, t);
   }
 }
 

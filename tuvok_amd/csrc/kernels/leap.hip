@@ -527,51 +527,34 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
   if (A.counter && ns) atomicAdd(A.counter, (unsigned long long)ns);
 }
 
-// one 8x8 tile per wave of the grid
+// persistent grid: every wave pulls 8x8 tiles from its XCD's chunk of the frame,
+// then from the others' (pull_tiles)
 template <int MODE, bool LIT, typename T>
 __global__ __launch_bounds__(256) void leap_kernel(LeapArgs A) {
-  leap_tile<MODE, LIT, T>(A, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
-}
-
-// persistent grid: every wave pulls 8x8 tiles from A.queue until tiles
-// 0 .. ntiles-1 are drained (every wave reaches that exit; the counter keeps
-// growing past ntiles: harmless)
-template <int MODE, bool LIT, typename T>
-__global__ __launch_bounds__(256) void leap_kernel_queue(LeapArgs A) {
   const int lane = threadIdx.x & 63;
-  for (;;) {
-    uint32_t t = 0;
-    if (lane == 0) t = atomicAdd(A.queue, 1u);
-    t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
-    if (t >= A.ntiles) break;
-    leap_tile<MODE, LIT, T>(A, t, lane);
-  }
+  pull_tiles(A.queues, A.xcd_items,
+             [&](uint32_t x, uint32_t t) { leap_tile<MODE, LIT, T>(A, x * A.xcd_items[0] + t, lane); });
 }
 
 template <int M, bool L, typename T>
 void launch_leap_one(const LeapArgs& a, uint32_t blocks, hipStream_t st) {
-  if (a.queue) {
-    // persistent grid: the workgroups the device holds at once
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(leap_kernel_queue<M, L, T>), 256, 0) != hipSuccess || per_cu <= 0)
-      per_cu = 1;
-    blocks = std::min(blocks, (uint32_t)per_cu * (uint32_t)cus);
-    hipLaunchKernelGGL((leap_kernel_queue<M, L, T>), dim3(blocks), dim3(256), 0, st, a);
-  } else {
-    hipLaunchKernelGGL((leap_kernel<M, L, T>), dim3(blocks), dim3(256), 0, st, a);
-  }
+  // the workgroups the device holds at once, no more than the tiles keep busy,
+  // a multiple of 8
+  int dev = 0, cus = 0, per_cu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(leap_kernel<M, L, T>), 256,
+                                                   0) != hipSuccess || per_cu <= 0)
+    per_cu = 1;
+  blocks = std::min(blocks, ((uint32_t)per_cu * (uint32_t)cus + 7u) & ~7u);
+  hipLaunchKernelGGL((leap_kernel<M, L, T>), dim3(blocks), dim3(256), 0, st, a);
 }
 
 }  // namespace
 
 hipError_t launch_leap(const LeapArgs& a, int bpv, hipStream_t st) {
-  const uint32_t tiles_y = ((uint32_t)a.H + 7u) / 8u;
-  const uint32_t tiles = a.tiles_x * tiles_y;
-  const uint32_t blocks = (tiles + 3u) / 4u;
+  const uint32_t blocks = (a.xcd_items[0] + 3u) / 4u * 8u;   // four tiles a workgroup, every XCD alike
   if (blocks == 0) return hipSuccess;
   const bool u16 = bpv == 2, lit = a.lighting != 0;
   if (a.mode == 0) {

@@ -23,6 +23,7 @@
 // ones of the host planner and of the reference restatement, in the same
 // order, so step counts, sample positions and TF indices are reproducible.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <type_traits>
 #include "../tvk_types.hpp"
 #include "stepnet.hpp"
@@ -382,12 +383,21 @@ struct CrossSampler<T, true> {
     nbx = nblocks((uint32_t)nx, Blk<T>::LX);
     nbxy = nbx * nblocks((uint32_t)ny, 2);
     const int xs = ic[0] - 1, sx = xs & ((1 << Blk<T>::LX) - 1);
+    // the four loads are issued before the first of them is used: near 128 VGPRs
+    // the scheduler otherwise waits for each in turn to save registers (64.0
+    // against 54.2 ms for 16 lit 2D 1080p frames of 1024^3)
+    typename Run4<T>::Word w[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) w[j][k] = run4_load<T>(base(), rowo(xs, ic[1] + j, ic[2] + k), sx);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         uint32_t v[4];
-        run4<T>(base(), rowo(xs, ic[1] + j, ic[2] + k), sx, v);
+        run4_take<T>(w[j][k], sx, v);
         xl[j][k] = (float)v[0];
         c[0][j][k] = (float)v[1];
         c[1][j][k] = (float)v[2];
@@ -1134,9 +1144,9 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
 // With work queues (A.queues, cleared to 0 before the launch) the grid is
 // persistent: every wave pulls 8x8 tiles -- item t of XCD x's queue is
 // quarter t & 3 of group order[xcd_start[x] + (t >> 2)] (or that index) --
-// first from its own XCD's queue, then from the others in turn, and exits when
-// all 8 are drained (every wave reaches that exit).  A wave that draws a light
-// tile comes back for another at once instead of waiting for its workgroup.
+// first from its own XCD's queue, then from the others (pull_tiles).  A wave
+// that draws a light tile comes back for another at once instead of waiting for
+// its workgroup.
 template <int MODE, bool LIT, typename T, bool COUNT, int LEARN>
 __device__ __forceinline__ void march_group(const MarchArgs& A) {
   extern __shared__ float4 s_tf[];  // 1D TF (tf_n entries, MODE 0 only)
@@ -1144,7 +1154,7 @@ __device__ __forceinline__ void march_group(const MarchArgs& A) {
   __shared__ uint64_t s_cols[MODE == 1 ? 4 * 64 : 1];                          // 2D TF column masks, one slice per wave
 
   const uint32_t lin = blockIdx.x, xcd = lin & 7u, j = lin >> 3;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
   // renders quarter q (x = q & 1, y = q >> 1) of 16x16 group g with this wave
   auto tile = [&](uint32_t g, int q) {
     int v = 0;
@@ -1175,34 +1185,25 @@ __device__ __forceinline__ void march_group(const MarchArgs& A) {
     for (int i = threadIdx.x; i < A.S.tf_n; i += 256) s_tf[i] = A.S.tf1[i];
     __syncthreads();   // the only workgroup barrier: the waves run independently after it
   }
-  uint32_t k = 0;   // queues tried so far, starting with this XCD's own
-  for (int it = 0;; ++it) {
-    uint32_t g;
-    int q;
-    if (A.queues == nullptr) {
-      if (it > 0) return;
-      g = g0;
-      q = wave;
-    } else {
-      uint32_t t = 0, x = 0;
-      for (; k < 8; ++k) {
-        x = (xcd + k) & 7u;
-        uint32_t tt = 0;
-        if (lane == 0) tt = atomicAdd(&A.queues[x], 1u);
-        tt = (uint32_t)__builtin_amdgcn_readfirstlane((int)tt);
-        if (tt < A.xcd_count[x] * 4u) { t = tt; break; }   // else drained (the counter grows past it: harmless)
-      }
-      if (k == 8) return;
+  // one call site for both launches: without queues the wave's single tile is
+  // the item of a queue that holds nothing else
+  pull_tiles(A.queues, A.xcd_items, [&](uint32_t x, uint32_t t) {
+    uint32_t g = g0;
+    int q = wave;
+    if (A.queues != nullptr) {
       const uint32_t gi = A.xcd_start[x] + (t >> 2);
       g = A.order ? (uint32_t)__builtin_amdgcn_readfirstlane((int)A.order[gi]) : gi;
       q = (int)(t & 3u);
     }
     tile(g, q);
-  }
+  });
 }
 
+// The fixed-step 2D and isosurface variants fit 128 VGPRs, 4 waves per SIMD,
+// without a spill; asked for, since the scheduler otherwise takes up to 151
+// (3 waves: 59.4 against 52.6 ms for 16 lit 2D 1080p frames of 1024^3).
 template <int MODE, bool LIT, typename T, bool COUNT, int LEARN>
-__global__ __launch_bounds__(256) void march_kernel(MarchArgs A) {
+__global__ __launch_bounds__(256, (LEARN == 0 && MODE != 0) ? 4 : 1) void march_kernel(MarchArgs A) {
   march_group<MODE, LIT, T, COUNT, LEARN>(A);
 }
 
@@ -1231,36 +1232,102 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void b
     BatchArgs B, const BatchRequest* __restrict__ req) {
   __shared__ __align__(16) uint16_t s_sn[LEARN > 0 ? 4 * SN_WAVE_LDS : 8];
   __shared__ uint64_t s_cols[MODE == 1 ? 4 * 64 : 1];
-  const uint32_t xcd = blockIdx.x & 7u;
-  const uint32_t chunk = (B.tiles_total + 7u) >> 3;
-  const int lane = threadIdx.x & 63;
-  for (uint32_t k = 0; k < 8; ++k) {
-    const uint32_t q = (xcd + k) & 7u;
-    const uint32_t lo = q * chunk, hi = min(B.tiles_total, lo + chunk);
-    if (lo >= hi) continue;
-    for (;;) {
-      uint32_t t = 0;
-      if (lane == 0) t = atomicAdd(&B.queues[q], 1u);
-      t = (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
-      t += lo;
-      if (t >= hi) break;   // this chunk is drained (the counter keeps growing past it: harmless)
-      // request of tile t: last request whose tile_offset <= t
-      int r0 = 0, r1 = B.nreq - 1;
-      while (r0 < r1) {
-        const int m = (r0 + r1 + 1) >> 1;
-        if (req[m].tile_offset <= t) r0 = m; else r1 = m - 1;
-      }
-      const BatchRequest* R = &req[__builtin_amdgcn_readfirstlane(r0)];
-      const uint32_t lt = t - R->tile_offset;
-      const uint32_t ty = lt / R->tiles_x, tx = lt - ty * R->tiles_x;
-      march_tile<MODE, LIT, T, COUNT, LEARN>(R->S, R->S.tf1, &R->V, B.list + R->V.list_offset, B.out,
-                                             (int)(tx * B.tile_w), (int)(ty * B.tile_h), (int)B.tile_w,
-                                             (int)B.tile_h, B.counter, (COUNT && B.touched) ? B.touched + R->touched_offset : nullptr,
-                                             &B.learn, nullptr, s_sn + (LEARN > 0 ? (threadIdx.x >> 6) * SN_WAVE_LDS : 0),
-                                             0u, s_cols + (MODE == 1 ? (threadIdx.x >> 6) * 64 : 0));
+  pull_tiles(B.queues, B.xcd_items, [&](uint32_t x, uint32_t i) {
+    const uint32_t t = x * B.xcd_items[0] + i;   // the chunks are equal but for the last
+    // request of tile t: last request whose tile_offset <= t
+    int r0 = 0, r1 = B.nreq - 1;
+    while (r0 < r1) {
+      const int m = (r0 + r1 + 1) >> 1;
+      if (req[m].tile_offset <= t) r0 = m; else r1 = m - 1;
+    }
+    const BatchRequest* R = &req[__builtin_amdgcn_readfirstlane(r0)];
+    const uint32_t lt = t - R->tile_offset;
+    const uint32_t ty = lt / R->tiles_x, tx = lt - ty * R->tiles_x;
+    march_tile<MODE, LIT, T, COUNT, LEARN>(R->S, R->S.tf1, &R->V, B.list + R->V.list_offset, B.out,
+                                           (int)(tx * B.tile_w), (int)(ty * B.tile_h), (int)B.tile_w,
+                                           (int)B.tile_h, B.counter, (COUNT && B.touched) ? B.touched + R->touched_offset : nullptr,
+                                           &B.learn, nullptr, s_sn + (LEARN > 0 ? (threadIdx.x >> 6) * SN_WAVE_LDS : 0),
+                                           0u, s_cols + (MODE == 1 ? (threadIdx.x >> 6) * 64 : 0));
+  });
+}
+
+// host-side launchers (extern "C++" within the library)
+
+// Persistent grid of a kernel: the workgroups the device holds at once (its
+// occupancy at this LDS size times the CU count), a multiple of 8 XCDs.
+static uint32_t persistent_grid(const void* kernel, size_t lds) {
+  int dev = 0, cus = 0, per_cu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, lds) != hipSuccess || per_cu <= 0) per_cu = 1;
+  const uint32_t n = (uint32_t)per_cu * (uint32_t)cus;
+  return (n + 7u) & ~7u;
+}
+
+template <typename K>
+static void launch_k(K kernel, const MarchArgs& a, size_t lds, hipStream_t st) {
+  // a queued frame with fewer 16x16 groups than the device holds workgroups
+  // takes one workgroup per group (groups_padded, a multiple of 8)
+  uint32_t grid = a.groups_padded;
+  if (a.queues) grid = std::min(grid, persistent_grid(reinterpret_cast<const void*>(kernel), lds));
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, st, a);
+}
+
+template <int M, bool L, typename T>
+static void launch_one(const MarchArgs& a, size_t lds, hipStream_t st, int learn) {
+  if constexpr (M != 2) {
+    if (learn == 2) return launch_k(march_kernel<M, L, T, false, 2>, a, lds, st);
+    if (learn == 1) {
+      if (a.counter) return launch_k(march_kernel_learn<M, L, T, true>, a, lds, st);
+      return launch_k(march_kernel_learn<M, L, T, false>, a, lds, st);
     }
   }
+  if (a.counter) return launch_k(march_kernel<M, L, T, true, 0>, a, lds, st);
+  launch_k(march_kernel<M, L, T, false, 0>, a, lds, st);
 }
+
+// The batch kernel's instance for a launch (learn as in launch_one).
+typedef void (*BatchKernel)(BatchArgs, const BatchRequest*);
+template <int M, bool L, typename T>
+static BatchKernel batch_instance(bool count, int learn) {
+  if constexpr (M != 2) {
+    if (learn == 1) return count ? batch_kernel<M, L, T, true, 1> : batch_kernel<M, L, T, false, 1>;
+  }
+  return count ? batch_kernel<M, L, T, true, 0> : batch_kernel<M, L, T, false, 0>;
+}
+
+// Everything of one render mode; this file is compiled once per mode
+// (TVK_MARCH_MODE), so that the modes' kernels build side by side.
+template <int M>
+void launch_march_mode(const MarchArgs& a, bool lit, bool u16, size_t lds, hipStream_t st, int learn) {
+  if constexpr (M != 2) {
+    if (lit) {
+      if (u16) launch_one<M, true, uint16_t>(a, lds, st, learn); else launch_one<M, true, uint8_t>(a, lds, st, learn);
+      return;
+    }
+  }
+  if (u16) launch_one<M, false, uint16_t>(a, lds, st, learn); else launch_one<M, false, uint8_t>(a, lds, st, learn);
+}
+template <int M>
+BatchKernel batch_kernel_mode(bool lit, bool u16, bool count, int learn) {
+  if constexpr (M != 2) {
+    if (lit) return u16 ? batch_instance<M, true, uint16_t>(count, learn) : batch_instance<M, true, uint8_t>(count, learn);
+  }
+  return u16 ? batch_instance<M, false, uint16_t>(count, learn) : batch_instance<M, false, uint8_t>(count, learn);
+}
+
+#ifndef TVK_MARCH_MODE
+#error "compile march.hip once per render mode: -DTVK_MARCH_MODE=0, 1, 2"
+#endif
+template void launch_march_mode<TVK_MARCH_MODE>(const MarchArgs&, bool, bool, size_t, hipStream_t, int);
+template BatchKernel batch_kernel_mode<TVK_MARCH_MODE>(bool, bool, bool, int);
+
+#if TVK_MARCH_MODE == 0
+extern template void launch_march_mode<1>(const MarchArgs&, bool, bool, size_t, hipStream_t, int);
+extern template void launch_march_mode<2>(const MarchArgs&, bool, bool, size_t, hipStream_t, int);
+extern template BatchKernel batch_kernel_mode<1>(bool, bool, bool, int);
+extern template BatchKernel batch_kernel_mode<2>(bool, bool, bool, int);
 
 __global__ void fill_u32(unsigned int* p, unsigned int n, unsigned int v) {
   const unsigned int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1273,125 +1340,40 @@ hipError_t launch_fill_u32(unsigned int* p, unsigned int n, unsigned int v, hipS
   return hipGetLastError();
 }
 
-// host-side launchers (extern "C++" within the library)
-
-// Persistent grid of a kernel: the workgroups the device holds at once (its
-// occupancy at this LDS size times the CU count), a multiple of 8 XCDs.
-static dim3 persistent_grid(const void* kernel, size_t lds) {
-  int dev = 0, cus = 0, per_cu = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, lds) != hipSuccess || per_cu <= 0) per_cu = 1;
-  const uint32_t n = (uint32_t)per_cu * (uint32_t)cus;
-  return dim3((n + 7u) & ~7u);
-}
-
-template <typename K>
-static void launch_k(K kernel, const MarchArgs& a, dim3 grid, size_t lds, hipStream_t st) {
-  if (a.queues) grid = persistent_grid(reinterpret_cast<const void*>(kernel), lds);
-  hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, a);
-}
-
-template <int M, bool L, typename T>
-static void launch_one(const MarchArgs& a, dim3 grid, size_t lds, hipStream_t st, int learn) {
-  if (learn == 2 && M != 2)
-    launch_k(march_kernel<M, L, T, false, (M != 2 ? 2 : 0)>, a, grid, lds, st);
-  else if (learn == 1 && M != 2) {
-    if (a.counter)
-      launch_k(march_kernel_learn<M, L, T, true>, a, grid, lds, st);
-    else
-      launch_k(march_kernel_learn<M, L, T, false>, a, grid, lds, st);
-  } else if (a.counter)
-    launch_k(march_kernel<M, L, T, true, 0>, a, grid, lds, st);
-  else
-    launch_k(march_kernel<M, L, T, false, 0>, a, grid, lds, st);
-}
-
 // learn: 0 fixed step, 1 step proposal (a.learn), 2 fixed step recording segment samples (a.seg)
-hipError_t launch_march(const MarchArgs& a, int bpv, hipStream_t st, int learn) {
-  dim3 grid(a.groups_padded);
+hipError_t launch_march(const MarchArgs& args, int bpv, hipStream_t st, int learn) {
+  MarchArgs a = args;
   const size_t lds = a.mode == 0 ? (size_t)a.S.tf_n * sizeof(float4) : 0;
-  const bool lit = a.lighting != 0 && a.mode != 2;
-  const bool u16 = bpv == 2;
-  if (learn != 0 && a.mode == 2) return hipErrorInvalidValue;
-  switch (a.mode) {
-    case 0:
-      if (lit) { if (u16) launch_one<0, true, uint16_t>(a, grid, lds, st, learn); else launch_one<0, true, uint8_t>(a, grid, lds, st, learn); }
-      else { if (u16) launch_one<0, false, uint16_t>(a, grid, lds, st, learn); else launch_one<0, false, uint8_t>(a, grid, lds, st, learn); }
-      break;
-    case 1:
-      if (lit) { if (u16) launch_one<1, true, uint16_t>(a, grid, lds, st, learn); else launch_one<1, true, uint8_t>(a, grid, lds, st, learn); }
-      else { if (u16) launch_one<1, false, uint16_t>(a, grid, lds, st, learn); else launch_one<1, false, uint8_t>(a, grid, lds, st, learn); }
-      break;
-    case 2:
-      if (u16) launch_one<2, false, uint16_t>(a, grid, lds, st, 0); else launch_one<2, false, uint8_t>(a, grid, lds, st, 0);
-      break;
-    default:
-      return hipErrorInvalidValue;
-  }
+  const bool lit = a.lighting != 0, u16 = bpv == 2;
+  if (a.mode < 0 || a.mode > 2 || (learn != 0 && a.mode == 2)) return hipErrorInvalidValue;
+  for (int x = 0; x < 8; ++x) a.xcd_items[x] = a.queues ? 4u * a.xcd_count[x] : a.groups_padded / 2u;
+  if (a.mode == 0) launch_march_mode<0>(a, lit, u16, lds, st, learn);
+  else if (a.mode == 1) launch_march_mode<1>(a, lit, u16, lds, st, learn);
+  else launch_march_mode<2>(a, lit, u16, lds, st, 0);
   return hipGetLastError();
 }
 
-template <int M, bool L, typename T>
-static void launch_batch_one(const BatchArgs& b, int groups, hipStream_t st, int learn) {
-  if (learn == 1 && M != 2) {
-    if (b.counter)
-      hipLaunchKernelGGL((batch_kernel<M, L, T, true, (M != 2 ? 1 : 0)>), dim3(groups), dim3(256), 0, st, b, b.req);
-    else
-      hipLaunchKernelGGL((batch_kernel<M, L, T, false, (M != 2 ? 1 : 0)>), dim3(groups), dim3(256), 0, st, b, b.req);
-  } else if (b.counter)
-    hipLaunchKernelGGL((batch_kernel<M, L, T, true, 0>), dim3(groups), dim3(256), 0, st, b, b.req);
-  else
-    hipLaunchKernelGGL((batch_kernel<M, L, T, false, 0>), dim3(groups), dim3(256), 0, st, b, b.req);
-}
-
-// occupancy of the exact instance launch_batch_one picks
-template <int M, bool L, typename T>
-static hipError_t occ_one(int* n, bool count, int learn) {
-  if (learn == 1 && M != 2)
-    return count ? hipOccupancyMaxActiveBlocksPerMultiprocessor(n, batch_kernel<M, L, T, true, (M != 2 ? 1 : 0)>, 256, 0)
-                 : hipOccupancyMaxActiveBlocksPerMultiprocessor(n, batch_kernel<M, L, T, false, (M != 2 ? 1 : 0)>, 256, 0);
-  return count ? hipOccupancyMaxActiveBlocksPerMultiprocessor(n, batch_kernel<M, L, T, true, 0>, 256, 0)
-               : hipOccupancyMaxActiveBlocksPerMultiprocessor(n, batch_kernel<M, L, T, false, 0>, 256, 0);
+static BatchKernel batch_kernel_of(int mode, bool lit, int bpv, bool count, int learn) {
+  const bool u16 = bpv == 2;
+  if (mode == 0) return batch_kernel_mode<0>(lit, u16, count, learn);
+  return mode == 1 ? batch_kernel_mode<1>(lit, u16, count, learn) : batch_kernel_mode<2>(lit, u16, count, 0);
 }
 
 // workgroups of the persistent kernel that fit on one CU at once
 int batch_occupancy(int mode, bool lit, int bpv, bool c, int l, int* n) {
-  const bool u16 = bpv == 2;
-  lit = lit && mode != 2;
-  if (mode == 2) l = 0;
-  if (mode == 0) return lit ? (u16 ? occ_one<0, true, uint16_t>(n, c, l) : occ_one<0, true, uint8_t>(n, c, l))
-                            : (u16 ? occ_one<0, false, uint16_t>(n, c, l) : occ_one<0, false, uint8_t>(n, c, l));
-  if (mode == 1) return lit ? (u16 ? occ_one<1, true, uint16_t>(n, c, l) : occ_one<1, true, uint8_t>(n, c, l))
-                            : (u16 ? occ_one<1, false, uint16_t>(n, c, l) : occ_one<1, false, uint8_t>(n, c, l));
-  return u16 ? occ_one<2, false, uint16_t>(n, c, 0) : occ_one<2, false, uint8_t>(n, c, 0);
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      n, reinterpret_cast<const void*>(batch_kernel_of(mode, lit, bpv, c, l)), 256, 0);
 }
 
-// Clears the 8 queue counters with a kernel (graph-capturable) and launches the
+// Clears the queue counters with a kernel (graph-capturable) and launches the
 // persistent kernel with `groups` workgroups.
 hipError_t launch_batch(const BatchArgs& b, int mode, bool lit, int bpv, int groups, hipStream_t st, int learn) {
-  hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, st, b.queues, 8u, 0u);
+  hipLaunchKernelGGL(fill_u32, dim3(1), dim3(QUEUE_WORDS), 0, st, b.queues, QUEUE_WORDS, 0u);
   if (b.tiles_total == 0 || groups <= 0) return hipGetLastError();
-  const bool u16 = bpv == 2;
-  lit = lit && mode != 2;
-  if (learn != 0 && mode == 2) learn = 0;
-  switch (mode) {
-    case 0:
-      if (lit) { if (u16) launch_batch_one<0, true, uint16_t>(b, groups, st, learn); else launch_batch_one<0, true, uint8_t>(b, groups, st, learn); }
-      else { if (u16) launch_batch_one<0, false, uint16_t>(b, groups, st, learn); else launch_batch_one<0, false, uint8_t>(b, groups, st, learn); }
-      break;
-    case 1:
-      if (lit) { if (u16) launch_batch_one<1, true, uint16_t>(b, groups, st, learn); else launch_batch_one<1, true, uint8_t>(b, groups, st, learn); }
-      else { if (u16) launch_batch_one<1, false, uint16_t>(b, groups, st, learn); else launch_batch_one<1, false, uint8_t>(b, groups, st, learn); }
-      break;
-    case 2:
-      if (u16) launch_batch_one<2, false, uint16_t>(b, groups, st, 0); else launch_batch_one<2, false, uint8_t>(b, groups, st, 0);
-      break;
-    default:
-      return hipErrorInvalidValue;
-  }
+  if (mode < 0 || mode > 2) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(batch_kernel_of(mode, lit, bpv, b.counter != nullptr, learn), dim3(groups), dim3(256), 0, st, b, b.req);
   return hipGetLastError();
 }
+#endif  // TVK_MARCH_MODE == 0
 
 }  // namespace tvk

@@ -356,13 +356,14 @@ int tvk_leap_render(tvk_ctx* c, int first, float* host_out, tvk_leap_stats* st) 
   a.tiles_x = (V.W + 7u) / 8u;
   a.ntiles = a.tiles_x * ((V.H + 7u) / 8u);
   {
-    // persistent launch: waves pull 8x8 tiles from one queue (a wave whose
+    // persistent launch: waves pull 8x8 tiles from the XCDs' queues (a wave whose
     // tile finishes early takes another instead of idling: 6.3 -> 5.6 ms for
     // a 1080p pass over the 1024^3 volume's pyramid)
-    int rc = ensure(c, &c->d_queues, &c->queues_cap, 8);
+    int rc = ensure(c, &c->d_queues, &c->queues_cap, QUEUE_WORDS);
     if (rc) return rc;
-    HIPCHK(c, launch_fill_u32(c->d_queues, 1u, 0u, c->stream));
-    a.queue = c->d_queues;
+    HIPCHK(c, launch_fill_u32(c->d_queues, QUEUE_WORDS, 0u, c->stream));
+    a.queues = c->d_queues;
+    chunk_items(a.ntiles, a.xcd_items);
   }
   if (c->count) HIPCHK(c, hipMemsetAsync(c->d_counter, 0, sizeof(unsigned long long), c->stream));
   HIPCHK(c, hipEventRecord(c->ev[6], c->stream));

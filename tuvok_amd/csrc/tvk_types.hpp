@@ -155,6 +155,10 @@ struct SegOut {
   uint32_t seed;
 };
 
+// Per-XCD work queues of the persistent launches (pull_tiles, kernels/common.hpp):
+// one counter per XCD, each in a 128-byte line of its own.
+constexpr uint32_t QUEUE_STRIDE = 32, QUEUE_WORDS = 8 * QUEUE_STRIDE;
+
 struct MarchArgs {
   ShadeConst S;
   LearnConst learn;
@@ -174,10 +178,11 @@ struct MarchArgs {
   // xcd_count[x] and groups_padded is 8 x the largest count.
   const uint32_t* order;
   uint32_t xcd_start[8], xcd_count[8];
-  // Work queues (or nullptr): 8 counters cleared before the launch; the grid
-  // is then persistent and every wave pulls 8x8 tiles, item t of XCD x being
-  // quarter t & 3 of the range's group t >> 2 (xcd_start / xcd_count as above,
-  // in the order when there is one).
+  uint32_t xcd_items[8];        // tiles of each XCD's queue (4 xcd_count; without queues one per wave)
+  // Work queues (or nullptr): QUEUE_WORDS words cleared before the launch; the
+  // grid is then persistent and every wave pulls 8x8 tiles, item t of XCD x
+  // being quarter t & 3 of the range's group t >> 2 (xcd_start / xcd_count as
+  // above, in the order when there is one).
   unsigned int* queues;
   int accumulate;               // continue the pixels' values (and depths) of an earlier launch
   float* depth;                 // isosurface: per-pixel depth of the best hit so far (or nullptr)
@@ -196,17 +201,18 @@ struct BatchRequest {
 
 // Persistent batch launch: waves pull tiles from 8 per-XCD queues (the tile
 // space is cut into 8 contiguous chunks; a wave drains its own XCD's chunk, then
-// the others in turn) and exit once every chunk is exhausted.
+// the others) and exit once every chunk is exhausted.
 struct BatchArgs {
   LearnConst learn;
   const BatchRequest* req;
   const FrameBrick* list;
   float* out;
-  unsigned int* queues;         // 8 counters, cleared by a fill kernel before the launch
+  unsigned int* queues;         // QUEUE_WORDS words, cleared by a fill kernel before the launch
   unsigned long long* counter;  // composited-sample counter or nullptr
   uint32_t* touched;            // per request: touched_offset + toc (or nullptr)
   int nreq;
   uint32_t tiles_total;
+  uint32_t xcd_items[8];        // tiles of each XCD's chunk: ceil(tiles_total / 8), the last ones what is left
   uint32_t tile_w, tile_h;      // wave tile shape, tile_w * tile_h == 64
 };
 
@@ -234,10 +240,16 @@ struct LeapArgs {
   float lod_factor, l0err, srm;
   int nlod, W, H, first, lighting, mode, overlap;
   uint32_t tiles_x;
-  // work queue (or nullptr: one 8x8 tile per wave of the grid): a counter
-  // cleared before the launch; the grid is then persistent and every wave
-  // pulls tiles 0 .. ntiles-1 in order until they are drained
-  unsigned int* queue;
+  // QUEUE_WORDS words cleared before the launch: the grid is persistent and its
+  // waves pull tiles 0 .. ntiles-1 in 8 contiguous chunks, one per XCD
+  unsigned int* queues;
   uint32_t ntiles;
+  uint32_t xcd_items[8];        // tiles of each XCD's chunk: ceil(ntiles / 8), the last ones what is left
 };
+
+// the 8 contiguous chunks of a persistent launch's n tiles
+inline void chunk_items(uint32_t n, uint32_t items[8]) {
+  const uint32_t per = (n + 7u) / 8u;
+  for (uint32_t x = 0; x < 8; ++x) items[x] = x * per < n ? (n - x * per < per ? n - x * per : per) : 0u;
+}
 }  // namespace tvk
