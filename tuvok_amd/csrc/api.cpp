@@ -744,8 +744,10 @@ int tvk_max_gradient(tvk_ctx* c, float* out) {
     // bricks' own overlap; a budgeted pool pages the bricks through its slots
     const LodInfo& l0 = c->L.lods[0];
     const uint32_t nb = (uint32_t)(l0.bricks[0] * l0.bricks[1] * l0.bricks[2]);
-    const uint32_t gx = 16;
     const uint32_t group = budgeted(c) ? c->pst->nslots : nb;
+    // workgroups per brick: about 8192 in all (several for each CU), so that a
+    // few large bricks fill the device as many small ones do
+    const uint32_t gx = std::min(512u, std::max(16u, 8192u / std::max(group, 1u)));
     GatherBrick* d_gb = nullptr;
     double* d_part = nullptr;
     HIPCHK(c, hipMalloc((void**)&d_gb, (size_t)group * sizeof(GatherBrick)));
