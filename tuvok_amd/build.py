@@ -34,6 +34,7 @@ SOURCES = [
     ("leap_api.cpp", ["-ffp-contract=off"]),
     ("noalloc.hip", ["-ffp-contract=off"]),
     ("pool.cpp", ["-ffp-contract=off"]),
+    ("devmem.cpp", []),
     ("host/tf2d.cpp", ["-ffp-contract=off"]),
     ("host/uvf.cpp", []),
 ]

@@ -43,8 +43,8 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
     return fail(c, TVK_ERR_UNSUPPORTED, "odd brick cores with coarser LODs need an overlap of at least 1");
   c->cp = tvk_ctx::CompatPool{};
   c->pool_bytes = (size_t)L.pool_elems * bpv;
-  HIPCHK(c, hipMalloc(&c->d_pool, c->pool_bytes));
-  c->pool_hold = std::shared_ptr<void>(c->d_pool, [](void* p) { (void)hipFree(p); });
+  HIPCHK(c, device_block(&c->pool_hold, c->pool_bytes));
+  c->d_pool = c->pool_hold.get();
   c->cells = std::make_shared<CellGrid>();
   // descriptors of every kept brick
   std::vector<GatherBrick> gb(L.toc.size());
@@ -52,10 +52,10 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
     for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)L.toc[i].coords[k]; gb[i].n[k] = L.toc[i].size[k]; }
     gb[i].offset = L.toc[i].offset;
   }
-  GatherBrick* d_gb = nullptr;
-  HIPCHK(c, hipMalloc(&d_gb, gb.size() * sizeof(GatherBrick)));
+  std::shared_ptr<void> gb_hold, mm_hold, snap_hold, tmp[2];
+  HIPCHK(c, device_block(&gb_hold, gb.size() * sizeof(GatherBrick)));
+  GatherBrick* d_gb = (GatherBrick*)gb_hold.get();
   HIPCHK(c, hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream));
-  void* tmp[2] = {nullptr, nullptr};
   const void* src = d_lin;
   int rc = TVK_OK;
   hipEvent_t ev[2] = {nullptr, nullptr};
@@ -65,8 +65,9 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
   // overlaps FillOverlap rewrites afterwards
   uint32_t* d_mm = nullptr;
   {
-    hipError_t e = hipMalloc(&d_mm, 2 * gb.size() * sizeof(uint32_t));
+    hipError_t e = device_block(&mm_hold, 2 * gb.size() * sizeof(uint32_t));
     if (e != hipSuccess) rc = hipfail(c, "hipMalloc(minmax)", e);
+    d_mm = (uint32_t*)mm_hold.get();
   }
   bool refilled = false;
   void* d_snap = nullptr;   // a level's bricks before FillOverlap (odd cores)
@@ -90,12 +91,13 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
     } else {
       if (lod > 0) {
         const uint64_t* sd = L.lods[lod - 1].size;
-        void*& dst = tmp[(lod - 1) % 2];
-        if (!dst) {
+        std::shared_ptr<void>& hold = tmp[(lod - 1) % 2];
+        if (!hold) {
           size_t bytes = (size_t)(li.size[0] * li.size[1] * li.size[2]) * bpv;
-          hipError_t e = hipMalloc(&dst, bytes);
+          hipError_t e = device_block(&hold, bytes);
           if (e != hipSuccess) { rc = hipfail(c, "hipMalloc(lod temp)", e); break; }
         }
+        void* const dst = hold.get();
         hipError_t e = launch_downsample(src, sd, dst, li.size, bpv, c->stream, c->lod_median);
         if (e != hipSuccess) { rc = hipfail(c, "downsample", e); break; }
         src = dst;
@@ -112,8 +114,9 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
         const TocBrick& last = L.toc[li.offset + nb - 1];
         snap_base = L.toc[li.offset].offset;
         const size_t bytes = (size_t)(last.offset + last.count - snap_base) * bpv;
-        if (d_snap) { (void)hipFree(d_snap); d_snap = nullptr; }
-        e = hipMalloc(&d_snap, bytes);
+        snap_hold.reset();
+        e = device_block(&snap_hold, bytes);
+        d_snap = snap_hold.get();
         if (e == hipSuccess)
           e = hipMemcpyAsync(d_snap, (uint8_t*)c->d_pool + snap_base * bpv, bytes, hipMemcpyDeviceToDevice,
                              c->stream);
@@ -133,8 +136,9 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
           }
       }
       start.push_back((uint32_t)order.size());
-      uint32_t* d_order = nullptr;
-      if (e == hipSuccess) e = hipMalloc(&d_order, order.size() * sizeof(uint32_t));
+      std::shared_ptr<void> order_hold;
+      if (e == hipSuccess) e = device_block(&order_hold, order.size() * sizeof(uint32_t));
+      uint32_t* const d_order = (uint32_t*)order_hold.get();
       if (e == hipSuccess)
         e = hipMemcpyAsync(d_order, order.data(), order.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
       uint32_t shell = 0;
@@ -148,7 +152,6 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
           e = launch_fill_overlap(c->d_pool, bpv, d_gb + li.offset, bxyz, L.overlap, d_order + start[w],
                                   start[w + 1] - start[w], shell, c->stream, d_snap, snap_base);
       if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-      if (d_order) (void)hipFree(d_order);
       if (e != hipSuccess) { rc = hipfail(c, "fill_overlap", e); break; }
     }
   }
@@ -176,10 +179,6 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
   if (ev[0] && ev[1] && rc == TVK_OK) (void)hipEventElapsedTime(&c->build_ms, ev[0], ev[1]);
   for (hipEvent_t e : ev)
     if (e) (void)hipEventDestroy(e);
-  if (d_mm) (void)hipFree(d_mm);
-  if (d_snap) (void)hipFree(d_snap);
-  (void)hipFree(d_gb);
-  for (void* t : tmp) if (t) (void)hipFree(t);
   if (rc != TVK_OK) return rc;
   c->minmax.resize(mm.size());
   for (size_t i = 0; i < mm.size(); ++i) c->minmax[i] = (double)mm[i];
@@ -296,14 +295,16 @@ int tvk_create(tvk_ctx** out, int device) {
     delete c;
     return TVK_ERR_HIP;
   }
+  device_hold(device);
   for (auto& ev : c->ev) (void)hipEventCreate(&ev);
   // this device's address of the allocation-free render's scratch array
   {
     const hipError_t se = scratch_address(device, &c->scratch);
     if (se != hipSuccess) c->scratch_err = std::string("hipGetSymbolAddress: ") + hipGetErrorString(se);
   }
-  if (hipMalloc(&c->d_counter, sizeof(unsigned long long)) != hipSuccess) {
+  if (device_alloc(&c->d_counter, sizeof(unsigned long long)) != hipSuccess) {
     delete c;
+    device_drop(device);
     return TVK_ERR_NOMEM;
   }
   *out = c;
@@ -336,7 +337,9 @@ void tvk_destroy(tvk_ctx* c) {
   if (c->h_order_pinned) (void)hipHostFree(c->h_order_pinned);
   for (auto& ev : c->ev) if (ev) (void)hipEventDestroy(ev);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  const int device = c->device;
   delete c;
+  device_drop(device);
 }
 
 const char* tvk_last_error(const tvk_ctx* c) { return c ? c->err.c_str() : "null context"; }
@@ -349,8 +352,8 @@ int tvk_load_volume(tvk_ctx* c, const void* host, int dtype, const uint64_t dims
   int rc = begin_dataset(c, dtype, dims, brick, overlap, clamp, max_lods);
   if (rc) return rc;
   const size_t bytes = (size_t)(dims[0] * dims[1] * dims[2]) * dtype;
-  HIPCHK(c, hipMalloc(&c->d_lin, bytes));
-  c->lin_hold = std::shared_ptr<void>(c->d_lin, [](void* p) { (void)hipFree(p); });
+  HIPCHK(c, device_block(&c->lin_hold, bytes));
+  c->d_lin = c->lin_hold.get();
   c->lin_bytes = bytes;
   HIPCHK(c, hipMemcpyAsync(c->d_lin, host, bytes, hipMemcpyHostToDevice, c->stream));
   rc = build_pool(c, c->d_lin);
@@ -371,8 +374,8 @@ int tvk_generate_volume(tvk_ctx* c, int kind, uint64_t seed, int dtype, const ui
   int rc = begin_dataset(c, dtype, dims, brick, overlap, clamp, max_lods);
   if (rc) return rc;
   const size_t bytes = (size_t)(dims[0] * dims[1] * dims[2]) * dtype;
-  HIPCHK(c, hipMalloc(&c->d_lin, bytes));
-  c->lin_hold = std::shared_ptr<void>(c->d_lin, [](void* p) { (void)hipFree(p); });
+  HIPCHK(c, device_block(&c->lin_hold, bytes));
+  c->d_lin = c->lin_hold.get();
   c->lin_bytes = bytes;
   SplitMix rng(seed);
   hipError_t e = hipSuccess;
@@ -388,7 +391,7 @@ int tvk_generate_volume(tvk_ctx* c, int kind, uint64_t seed, int dtype, const ui
       g.amp[b] = (float)rng.uniform(0.3, 1.0);
       g.inv2s2[b] = (float)(1.0 / (2.0 * sigma * sigma));
     }
-    e = hipMalloc(&d_tmp, sizeof(unsigned));
+    e = device_alloc(&d_tmp, sizeof(unsigned));
     if (e == hipSuccess) e = launch_blobs(g, dims, dtype, c->d_lin, d_tmp, seed, c->stream);
   } else if (kind == TVK_GEN_FBM_SHELLS) {
     // 3-octave value-noise fBm + 64 hollow shells (radius 0.02-0.1, 2 voxels thick, value 60000)
@@ -423,7 +426,7 @@ int tvk_generate_volume(tvk_ctx* c, int kind, uint64_t seed, int dtype, const ui
       }
       q.amin = std::min(q.a[0], std::min(q.a[1], q.a[2]));
     }
-    e = hipMalloc(&d_e, el.size() * sizeof(GenEllipsoid));
+    e = device_alloc(&d_e, el.size() * sizeof(GenEllipsoid));
     if (e == hipSuccess) e = hipMemcpyAsync(d_e, el.data(), el.size() * sizeof(GenEllipsoid), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) {
       if (kind == TVK_GEN_ELLIPSOID_SDF) {
@@ -520,7 +523,7 @@ int tvk_crop_dataset(tvk_ctx* c, int keep_old, float plane_used[4]) {
   const size_t bytes = (size_t)(L.dims[0] * L.dims[1] * L.dims[2]) * (size_t)L.bpv;
   if (!d_lin) {
     if (budgeted(c)) return fail(c, TVK_ERR_UNSUPPORTED, "cropping a budgeted dataset needs its linear volume");
-    HIPCHK(c, hipMalloc(&d_lin, bytes));
+    HIPCHK(c, device_alloc(&d_lin, bytes));
     lin = std::shared_ptr<void>(d_lin, [](void* p) { (void)hipFree(p); });
     const LodInfo& l0 = L.lods[0];
     std::vector<GatherBrick> gb((size_t)(l0.bricks[0] * l0.bricks[1] * l0.bricks[2]));
@@ -530,7 +533,7 @@ int tvk_crop_dataset(tvk_ctx* c, int keep_old, float plane_used[4]) {
       gb[i].offset = t.offset;
     }
     GatherBrick* d_gb = nullptr;
-    HIPCHK(c, hipMalloc((void**)&d_gb, gb.size() * sizeof(GatherBrick)));
+    HIPCHK(c, device_alloc((void**)&d_gb, gb.size() * sizeof(GatherBrick)));
     std::shared_ptr<void> gb_hold(d_gb, [](void* p) { (void)hipFree(p); });
     HIPCHK(c, hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream));
     const uint32_t nb[3] = {(uint32_t)l0.bricks[0], (uint32_t)l0.bricks[1], (uint32_t)l0.bricks[2]};
@@ -694,21 +697,19 @@ int download_ref(tvk_ctx* c, size_t first, size_t n, void* host, size_t bytes) {
     maxv = std::max<uint32_t>(maxv, (uint32_t)t.real);
   }
   if (bytes != total * (size_t)L.bpv) return fail(c, TVK_ERR_ARG, "size mismatch");
-  GatherBrick* d_gb = nullptr;
-  uint64_t* d_ro = nullptr;
-  void* d_out = nullptr;
-  hipError_t e = hipMalloc(&d_gb, n * sizeof(GatherBrick));
-  if (e == hipSuccess) e = hipMalloc(&d_ro, n * sizeof(uint64_t));
-  if (e == hipSuccess) e = hipMalloc(&d_out, bytes);
+  std::shared_ptr<void> gb_hold, ro_hold, out_hold;
+  hipError_t e = device_block(&gb_hold, n * sizeof(GatherBrick));
+  if (e == hipSuccess) e = device_block(&ro_hold, n * sizeof(uint64_t));
+  if (e == hipSuccess) e = device_block(&out_hold, bytes);
+  GatherBrick* const d_gb = (GatherBrick*)gb_hold.get();
+  uint64_t* const d_ro = (uint64_t*)ro_hold.get();
+  void* const d_out = out_hold.get();
   if (e == hipSuccess) e = hipMemcpyAsync(d_gb, gb.data(), n * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(d_ro, ro.data(), n * sizeof(uint64_t), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) e = launch_unswizzle(c->d_pool, L.bpv, d_gb, d_ro, (uint32_t)n, maxv, d_out, c->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(host, d_out, bytes, hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   (void)hipStreamSynchronize(c->stream);
-  if (d_gb) (void)hipFree(d_gb);
-  if (d_ro) (void)hipFree(d_ro);
-  if (d_out) (void)hipFree(d_out);
   if (e != hipSuccess) return hipfail(c, "brick download", e);
   return TVK_OK;
 }
@@ -748,12 +749,11 @@ int tvk_max_gradient(tvk_ctx* c, float* out) {
     // workgroups per brick: about 8192 in all (several for each CU), so that a
     // few large bricks fill the device as many small ones do
     const uint32_t gx = std::min(512u, std::max(16u, 8192u / std::max(group, 1u)));
-    GatherBrick* d_gb = nullptr;
-    double* d_part = nullptr;
-    HIPCHK(c, hipMalloc((void**)&d_gb, (size_t)group * sizeof(GatherBrick)));
-    std::shared_ptr<void> gb_hold(d_gb, [](void* p) { (void)hipFree(p); });
-    HIPCHK(c, hipMalloc((void**)&d_part, (size_t)group * gx * sizeof(double)));
-    std::shared_ptr<void> part_hold(d_part, [](void* p) { (void)hipFree(p); });
+    std::shared_ptr<void> gb_hold, part_hold;
+    HIPCHK(c, device_block(&gb_hold, (size_t)group * sizeof(GatherBrick)));
+    HIPCHK(c, device_block(&part_hold, (size_t)group * gx * sizeof(double)));
+    GatherBrick* const d_gb = (GatherBrick*)gb_hold.get();
+    double* const d_part = (double*)part_hold.get();
     double m = 0.0;
     std::vector<double> h((size_t)group * gx);
     for (uint32_t first = 0; first < nb; first += group) {
@@ -783,7 +783,7 @@ int tvk_max_gradient(tvk_ctx* c, float* out) {
   if (!c->d_lin) return fail(c, TVK_ERR_STATE, "without overlap the gradient needs the kept linear volume");
   const uint32_t blocks = 4096;
   double* d = nullptr;
-  HIPCHK(c, hipMalloc(&d, blocks * sizeof(double)));
+  HIPCHK(c, device_alloc(&d, blocks * sizeof(double)));
   std::vector<double> h(blocks);
   hipError_t e = launch_max_gradient(c->d_lin, c->L.bpv, c->L.dims, c->clamp, d, blocks, c->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d, blocks * sizeof(double), hipMemcpyDeviceToHost, c->stream);
@@ -1003,10 +1003,10 @@ int ensure_compat(tvk_ctx* c) {
   }
   const size_t bytes = (size_t)elems * (size_t)cp.bpv;
   c->cp = tvk_ctx::CompatPool{};   // the old textures go before the new ones are made
-  HIPCHK(c, hipMalloc(&cp.d, std::max<size_t>(bytes, 1)));
+  HIPCHK(c, device_alloc(&cp.d, std::max<size_t>(bytes, 1)));
   cp.hold = std::shared_ptr<void>(cp.d, [](void* p) { (void)hipFree(p); });
   GatherBrick* d_gb = nullptr;
-  HIPCHK(c, hipMalloc(&d_gb, 2 * nb * sizeof(GatherBrick)));
+  HIPCHK(c, device_alloc(&d_gb, 2 * nb * sizeof(GatherBrick)));
   hipError_t e = hipMemcpyAsync(d_gb, src.data(), nb * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(d_gb + nb, dst.data(), nb * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
@@ -1146,9 +1146,9 @@ int ensure_cells(tvk_ctx* c) {
   GatherBrick* d_gb = nullptr;
   uint32_t* d_base = nullptr;
   uint32_t* d_cells = nullptr;
-  hipError_t e = hipMalloc(&d_cells, std::max<uint64_t>(total, 1) * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMalloc(&d_gb, gb.size() * sizeof(GatherBrick));
-  if (e == hipSuccess) e = hipMalloc(&d_base, G.base.size() * sizeof(uint32_t));
+  hipError_t e = device_alloc(&d_cells, std::max<uint64_t>(total, 1) * sizeof(uint32_t));
+  if (e == hipSuccess) e = device_alloc(&d_gb, gb.size() * sizeof(GatherBrick));
+  if (e == hipSuccess) e = device_alloc(&d_base, G.base.size() * sizeof(uint32_t));
   if (e == hipSuccess)
     e = hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess)
@@ -1539,8 +1539,8 @@ int tvk_generate_segments(tvk_ctx* c, int nviews, const float* rots, uint32_t ca
   HIPCHK(c, hipSetDevice(c->device));
   SegSample* d_out = nullptr;
   unsigned int* d_cnt = nullptr;
-  HIPCHK(c, hipMalloc((void**)&d_out, (size_t)cap * sizeof(SegSample)));
-  hipError_t e = hipMalloc((void**)&d_cnt, sizeof(unsigned int));
+  HIPCHK(c, device_alloc((void**)&d_out, (size_t)cap * sizeof(SegSample)));
+  hipError_t e = device_alloc((void**)&d_cnt, sizeof(unsigned int));
   if (e == hipSuccess) e = hipMemsetAsync(d_cnt, 0, sizeof(unsigned int), c->stream);
   int rc = e == hipSuccess ? TVK_OK : hipfail(c, "segment buffers", e);
   if (!rc) {
@@ -1636,7 +1636,7 @@ int tvk_display(tvk_ctx* c, const float bg_top[3], const float bg_bottom[3], uin
   if (bytes != px * 4) return fail(c, TVK_ERR_ARG, "output size mismatch");
   HIPCHK(c, hipSetDevice(c->device));
   uint8_t* d = nullptr;
-  HIPCHK(c, hipMalloc((void**)&d, bytes));
+  HIPCHK(c, device_alloc((void**)&d, bytes));
   hipError_t e = launch_display(c->d_out, c->last_w, c->last_h, (uint32_t)c->last_views, bg_top, bg_bottom, d,
                                 c->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(out, d, bytes, hipMemcpyDeviceToHost, c->stream);

@@ -93,7 +93,7 @@ int bensure(tvk_batch* b, T** p, size_t* cap, size_t n) {
   if (*cap >= n && *p) return TVK_OK;
   if (*p) { (void)hipFree(*p); *p = nullptr; *cap = 0; }
   const size_t want = std::max<size_t>(n + n / 4, 1);
-  BCHK(b, hipMalloc((void**)p, want * sizeof(T)));
+  BCHK(b, device_alloc(p, want * sizeof(T)));
   *cap = want;
   return TVK_OK;
 }

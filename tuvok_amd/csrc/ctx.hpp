@@ -14,6 +14,7 @@
 #include "host/host.hpp"
 #include "kernels/generate.hpp"
 #include "tvk_types.hpp"
+#include "devmem.hpp"
 
 namespace tvk {
 hipError_t launch_march(const MarchArgs& a, int bpv, hipStream_t st, int learn);
@@ -251,7 +252,7 @@ int ensure(tvk_ctx* c, T** p, size_t* cap, size_t n) {
   if (*cap >= n && *p) return TVK_OK;
   if (*p) { (void)hipFree(*p); *p = nullptr; *cap = 0; }
   size_t want = std::max<size_t>(n, 1);
-  HIPCHK(c, hipMalloc((void**)p, want * sizeof(T)));
+  HIPCHK(c, device_alloc(p, want * sizeof(T)));
   *cap = want;
   return TVK_OK;
 }

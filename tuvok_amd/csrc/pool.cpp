@@ -84,7 +84,7 @@ int ensure_stage(tvk_ctx* c, PoolState& P, size_t bytes, size_t nb) {
     if (P.d_stage) (void)hipFree(P.d_stage);
     P.d_stage = nullptr;
     P.stage_bytes = 0;
-    HIPCHK(c, hipMalloc((void**)&P.d_stage, bytes));
+    HIPCHK(c, device_alloc((void**)&P.d_stage, bytes));
     P.stage_bytes = bytes;
   }
   if (P.desc_cap < nb) {
@@ -93,8 +93,8 @@ int ensure_stage(tvk_ctx* c, PoolState& P, size_t bytes, size_t nb) {
     P.d_desc = nullptr;
     P.d_srcoff = nullptr;
     P.desc_cap = 0;
-    HIPCHK(c, hipMalloc((void**)&P.d_desc, nb * sizeof(GatherBrick)));
-    HIPCHK(c, hipMalloc((void**)&P.d_srcoff, nb * sizeof(uint64_t)));
+    HIPCHK(c, device_alloc((void**)&P.d_desc, nb * sizeof(GatherBrick)));
+    HIPCHK(c, device_alloc((void**)&P.d_srcoff, nb * sizeof(uint64_t)));
     P.desc_cap = nb;
   }
   return TVK_OK;
@@ -258,7 +258,7 @@ int pool_set_budget(tvk_ctx* c, uint64_t budget) {
     for (size_t t = 0; t < nb; ++t)
       if (!P.present[t]) return fail(c, TVK_ERR_STATE, "not every brick was uploaded");
     void* full = nullptr;
-    HIPCHK(c, hipMalloc(&full, (size_t)L.pool_elems * bpv));
+    HIPCHK(c, device_alloc(&full, (size_t)L.pool_elems * bpv));
     std::shared_ptr<void> hold(full, [](void* p) { (void)hipFree(p); });
     std::vector<const uint8_t*> src(nb);
     std::vector<uint32_t> toc(nb);
@@ -299,13 +299,13 @@ int pool_set_budget(tvk_ctx* c, uint64_t budget) {
     size_t largest = 0;
     for (const TocBrick& b : L.toc) largest = std::max(largest, (size_t)b.real * bpv);
     const size_t tmp_bytes = std::max(largest, std::min(batch_bytes, (size_t)L.ref_elems * bpv));
-    HIPCHK(c, hipMalloc(&tmp, tmp_bytes));
+    HIPCHK(c, device_alloc(&tmp, tmp_bytes));
     std::shared_ptr<void> tmp_hold(tmp, [](void* p) { (void)hipFree(p); });
     GatherBrick* d_gb = nullptr;
     uint64_t* d_ro = nullptr;
-    HIPCHK(c, hipMalloc((void**)&d_gb, 65535 * sizeof(GatherBrick)));
+    HIPCHK(c, device_alloc((void**)&d_gb, 65535 * sizeof(GatherBrick)));
     std::shared_ptr<void> gb_hold(d_gb, [](void* p) { (void)hipFree(p); });
-    HIPCHK(c, hipMalloc((void**)&d_ro, 65535 * sizeof(uint64_t)));
+    HIPCHK(c, device_alloc((void**)&d_ro, 65535 * sizeof(uint64_t)));
     std::shared_ptr<void> ro_hold(d_ro, [](void* p) { (void)hipFree(p); });
     while (i < nb) {
       std::vector<GatherBrick> gb;
@@ -337,7 +337,7 @@ int pool_set_budget(tvk_ctx* c, uint64_t budget) {
     }
   }
   void* slots = nullptr;
-  HIPCHK(c, hipMalloc(&slots, (size_t)P->nslots * slot * bpv));
+  HIPCHK(c, device_alloc(&slots, (size_t)P->nslots * slot * bpv));
   P->slot_brick.assign(P->nslots, -1);
   P->slot_time.assign(P->nslots, 0);
   P->brick_slot.assign(nb, -1);
@@ -563,7 +563,7 @@ int tvk_set_bricks(tvk_ctx* c, int dtype, const uint64_t dims[3], const uint32_t
   const size_t full = (size_t)c->L.pool_elems * (size_t)dtype;
   if (budget == 0 || budget >= full) {
     // every brick resident at its TOC offset; uploads go straight to the pool
-    HIPCHK(c, hipMalloc(&c->d_pool, full));
+    HIPCHK(c, device_alloc(&c->d_pool, full));
     c->pool_hold = std::shared_ptr<void>(c->d_pool, [](void* p) { (void)hipFree(p); });
     c->pool_bytes = full;
     c->cells = std::make_shared<CellGrid>();
@@ -579,7 +579,7 @@ int tvk_set_bricks(tvk_ctx* c, int dtype, const uint64_t dims[3], const uint32_t
     int rc = alloc_store(c, *P);
     if (rc) return rc;
     void* slots = nullptr;
-    HIPCHK(c, hipMalloc(&slots, (size_t)P->nslots * slot * (size_t)dtype));
+    HIPCHK(c, device_alloc(&slots, (size_t)P->nslots * slot * (size_t)dtype));
     c->pool_hold = std::shared_ptr<void>(slots, [](void* p) { (void)hipFree(p); });
     c->d_pool = slots;
     c->pool_bytes = (size_t)P->nslots * slot * (size_t)dtype;

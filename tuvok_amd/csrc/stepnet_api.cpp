@@ -75,7 +75,7 @@ template <typename T>
 int sensure(tvk_stepnet* s, T** p, size_t* cap, size_t n) {
   if (*cap >= n && *p) return TVK_OK;
   if (*p) { (void)hipFree(*p); *p = nullptr; *cap = 0; }
-  SCHK(s, hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T)));
+  SCHK(s, device_alloc((void**)p, std::max<size_t>(n, 1) * sizeof(T)));
   *cap = std::max<size_t>(n, 1);
   return TVK_OK;
 }
@@ -117,13 +117,13 @@ int tvk_stepnet_create(tvk_stepnet** out, int device, uint64_t seed) {
   s->device = device;
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc((void**)&s->d_theta, SN_NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&s->d_m, SN_NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&s->d_v, SN_NPARAM * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&s->d_grad, (SN_NPARAM + 1) * sizeof(float));
+  if (e == hipSuccess) e = device_alloc((void**)&s->d_theta, SN_NPARAM * sizeof(float));
+  if (e == hipSuccess) e = device_alloc((void**)&s->d_m, SN_NPARAM * sizeof(float));
+  if (e == hipSuccess) e = device_alloc((void**)&s->d_v, SN_NPARAM * sizeof(float));
+  if (e == hipSuccess) e = device_alloc((void**)&s->d_grad, (SN_NPARAM + 1) * sizeof(float));
   if (e == hipSuccess)
-    e = hipMalloc((void**)&s->d_w, (SN_HID * SN_INP + 2 * SN_HID * SN_HID + 32 * SN_HID) * sizeof(uint16_t));
-  if (e == hipSuccess) e = hipMalloc((void**)&s->d_b, (2 * SN_HID + SN_OUT) * sizeof(float));
+    e = device_alloc((void**)&s->d_w, (SN_HID * SN_INP + 2 * SN_HID * SN_HID + 32 * SN_HID) * sizeof(uint16_t));
+  if (e == hipSuccess) e = device_alloc((void**)&s->d_b, (2 * SN_HID + SN_OUT) * sizeof(float));
   if (e != hipSuccess) {
     tvk_stepnet_destroy(s);
     return TVK_ERR_HIP;
@@ -201,9 +201,9 @@ int tvk_stepnet_set_data(tvk_stepnet* s, const float* feat, const float* tgt, in
     s->d_feat = s->d_tgt = nullptr;
     s->d_idx = nullptr;
     s->data_cap = 0;
-    SCHK(s, hipMalloc((void**)&s->d_feat, (size_t)n * SN_IN * sizeof(float)));
-    SCHK(s, hipMalloc((void**)&s->d_tgt, (size_t)n * 3 * sizeof(float)));
-    SCHK(s, hipMalloc((void**)&s->d_idx, (size_t)n * sizeof(uint32_t)));
+    SCHK(s, device_alloc((void**)&s->d_feat, (size_t)n * SN_IN * sizeof(float)));
+    SCHK(s, device_alloc((void**)&s->d_tgt, (size_t)n * 3 * sizeof(float)));
+    SCHK(s, device_alloc((void**)&s->d_idx, (size_t)n * sizeof(uint32_t)));
     s->data_cap = (size_t)n;
   }
   SCHK(s, hipMemcpyAsync(s->d_feat, feat, (size_t)n * SN_IN * sizeof(float), hipMemcpyHostToDevice, s->stream));
