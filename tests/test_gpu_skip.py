@@ -1,0 +1,108 @@
+"""The march that goes by stretches that cannot contribute (datasets with a cell
+grid) against the march that samples every step: a budgeted pool has no grid, so
+its frames, sample counts and hits must equal the resident pool's bit for bit."""
+import numpy as np
+import pytest
+
+from tuvok_amd import RM_1DTRANS, RM_ISOSURFACE, HIPRaycaster, RenderBatch, rotation_y
+
+pytestmark = pytest.mark.gpu
+
+
+def sparse_volume(dims, dtype, seed):
+    """Islands, thin sheets and single voxels in an empty volume, some at its faces."""
+    rng = np.random.default_rng(seed)
+    top = np.iinfo(dtype).max
+    v = np.zeros(dims[::-1], dtype)
+    for _ in range(6):
+        c = [int(rng.integers(0, n)) for n in dims]
+        r = [int(rng.integers(1, 9)) for _ in range(3)]
+        s = tuple(slice(max(0, c[a] - r[a]), c[a] + r[a]) for a in (2, 1, 0))
+        v[s] = rng.integers(top // 3, top, v[s].shape)
+    v[:, dims[1] // 2, :] = top // 2
+    for _ in range(20):
+        v[tuple(int(rng.integers(0, n)) for n in dims[::-1])] = top
+    return v
+
+
+def table(kind):
+    t = np.zeros((256, 4), np.uint8)
+    t[:, :3] = np.arange(256)[:, None]
+    t[:, 3] = {"ramp": np.maximum(np.arange(256) - 60, 0) // 2, "gaps": np.where(np.arange(256) % 64 > 50, 30, 0),
+               "all": 20, "last": np.where(np.arange(256) == 255, 200, 0)}[kind]
+    return t
+
+
+def frames(r, rots):
+    r.SetCountSamples(True)
+    f = r.PaintViews(rots)
+    n = r.last_stats.samples
+    r.SetCountSamples(False)
+    assert np.array_equal(f, r.PaintViews(rots))
+    return f, n
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16])
+@pytest.mark.parametrize("dims,brick,ov,edge", [((70, 53, 61), 18, 1, False), ((64, 64, 192), 66, 1, False),
+                                                ((45, 90, 33), 34, 2, True), ((40, 40, 40), 12, 0, False),
+                                                ((300, 3, 50), 130, 1, True)])
+def test_skipped_stretches(dims, brick, ov, edge, dtype):
+    vol = sparse_volume(dims, dtype, 7)
+    rots = [rotation_y(a) for a in (0.0, 0.7, 2.1)]
+    with HIPRaycaster(0) as r, HIPRaycaster(0) as q:
+        for x in (r, q):
+            x.LoadVolume(vol, (brick,) * 3, ov, clamp_to_edge=edge, max_lods=1)
+            x.SetClampToEdge(edge)
+            x.SetViewParameters(45.0, 0.01, 1000.0)
+            x.SetViewPosition((0.1, 0.2, 1.7))
+            x.Resize(97, 83)
+        q.SetPoolBudget(q.GetDatasetDesc().pool_bytes - 1)
+        for mode, tf, lit, srm, ert in ((RM_1DTRANS, "ramp", False, 1.0, 0.0), (RM_1DTRANS, "ramp", True, 2.0, 2.0 ** -11),
+                                        (RM_1DTRANS, "gaps", True, 1.0, 0.0), (RM_1DTRANS, "gaps", False, 0.7, 2.0 ** -11),
+                                        (RM_1DTRANS, "all", False, 1.0, 0.0), (RM_1DTRANS, "last", True, 1.0, 0.0),
+                                        (RM_ISOSURFACE, None, True, 1.0, 0.0), (RM_ISOSURFACE, None, True, 3.0, 2.0 ** -11)):
+            for x in (r, q):
+                if tf:
+                    x.Set1DTrans(table(tf))
+                x.SetRendermode(mode)
+                x.SetUseLighting(lit)
+                x.SetSampleRateModifier(srm)
+                x.SetEarlyRayTermination(ert)
+                x.SetIsoValue(np.iinfo(dtype).max * 0.4)
+            (a, na), (b, nb) = frames(r, rots), frames(q, rots)
+            assert np.array_equal(a, b), (mode, tf, lit, srm)
+            if mode == RM_1DTRANS or ert == 0.0:   # the hit skip of a frame rendered in parts sees only its part
+                assert na == nb
+            assert tf == "last" or a[..., 3].max() > 0   # only the very top value: samples may miss it
+
+
+def test_brick_uploaded_again_reaches_every_context():
+    """A brick of a shared dataset changes: the other context's next frame and a
+    batch see it, although both rendered (and skipped) with the old grid before."""
+    dims, brick = (32, 32, 32), 34
+    empty = np.zeros((34, 34, 34), np.uint8)
+    full = np.zeros((34, 34, 34), np.uint8)
+    full[10:20, 10:20, 10:20] = 255
+    with HIPRaycaster(0) as a, HIPRaycaster(0) as b:
+        a.SetBricks(np.uint8, dims, (brick,) * 3, 1, [(0, 0, (0.0, 255.0))], lod_count=1)
+        a.UploadBrick(0, 0, empty)
+        b.ShareDataset(a)
+        for x in (a, b):
+            x.Set1DTrans(table("ramp"))
+            x.SetRendermode(RM_1DTRANS)
+            x.SetUseLighting(False)
+            x.SetViewParameters(45.0, 0.01, 1000.0)
+            x.SetViewPosition((0.0, 0.0, 1.8))
+            x.Resize(64, 64)
+            assert x.Paint()[..., 3].max() == 0
+        batch = RenderBatch(0)
+        batch.Add(b, None, 64, 64)
+        batch.Render()
+        assert batch.Frame(0)[..., 3].max() == 0
+        a.UploadBrick(0, 0, full)
+        fb = b.Paint()
+        assert fb[..., 3].max() > 0.5
+        assert np.array_equal(fb, a.Paint())
+        batch.Render()
+        assert np.array_equal(batch.Frame(0), fb)
+        batch.close()

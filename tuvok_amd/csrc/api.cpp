@@ -69,6 +69,12 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
     if (e != hipSuccess) rc = hipfail(c, "hipMalloc(minmax)", e);
     d_mm = (uint32_t*)mm_hold.get();
   }
+  // ranges of every 4^3 voxels, written with the bricks (without room for them
+  // the cell grid is made on first use instead)
+  std::shared_ptr<void> quad_hold;
+  (void)device_block(&quad_hold, quad_words(L) * sizeof(uint32_t));
+  if (!quad_hold) (void)hipGetLastError();
+  uint32_t* const d_quads = (uint32_t*)quad_hold.get();
   bool refilled = false;
   void* d_snap = nullptr;   // a level's bricks before FillOverlap (odd cores)
   for (size_t lod = 0; lod < keep && rc == TVK_OK; ++lod) {
@@ -103,7 +109,7 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
         src = dst;
       }
       hipError_t e = launch_gather(src, bpv, li.size, d_gb + li.offset, nb, (uint32_t)li.bricks[0], maxv, c->d_pool,
-                                   core, L.overlap, c->clamp, d_mm + 2 * li.offset, c->stream);
+                                   core, L.overlap, c->clamp, d_mm + 2 * li.offset, d_quads, c->stream);
       if (e != hipSuccess) { rc = hipfail(c, "gather", e); break; }
     }
     if (lod > 0 && !c->clamp && nb > 1) {
@@ -163,7 +169,7 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
     for (size_t i = first; i < L.toc.size(); ++i) maxv = std::max<uint32_t>(maxv, (uint32_t)L.toc[i].count);
     hipError_t e = launch_extend(c->d_pool, bpv, d_gb + first, (uint32_t)(gb.size() - first), maxv, c->stream);
     if (e == hipSuccess)
-      e = launch_minmax(c->d_pool, bpv, d_gb + first, (uint32_t)(gb.size() - first), maxv, d_mm + 2 * first,
+      e = launch_minmax(c->d_pool, bpv, d_gb + first, (uint32_t)(gb.size() - first), maxv, d_mm + 2 * first, d_quads,
                         c->stream);
     if (e != hipSuccess) rc = hipfail(c, "extend/minmax", e);
   }
@@ -180,6 +186,11 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
   for (hipEvent_t e : ev)
     if (e) (void)hipEventDestroy(e);
   if (rc != TVK_OK) return rc;
+  if (d_quads) {
+    const std::string msg = c->err;
+    std::lock_guard<std::mutex> lk(c->cells->mu);
+    if (make_cells(c, *c->cells, d_quads) != TVK_OK) { (void)hipGetLastError(); c->err = msg; }   // marches go without it
+  }
   c->minmax.resize(mm.size());
   for (size_t i = 0; i < mm.size(); ++i) c->minmax[i] = (double)mm[i];
   // UVFDataset::ComputeRange over the LOD0 bricks (uvfDataset.cpp:1120-1165)
@@ -322,6 +333,7 @@ void tvk_destroy(tvk_ctx* c) {
   for (void* q : {(void*)c->d_leap_meta, (void*)c->d_leap_table, (void*)c->d_leap_bricks, (void*)c->d_leap_resume})
     if (q) (void)hipFree(q);
   if (c->d_tf1f) (void)hipFree(c->d_tf1f);
+  if (c->d_tf1next) (void)hipFree(c->d_tf1next);
   if (c->d_tf2cols) (void)hipFree(c->d_tf2cols);
   if (c->d_list) (void)hipFree(c->d_list);
   if (c->d_views) (void)hipFree(c->d_views);
@@ -804,11 +816,16 @@ int tvk_set_tf1d(tvk_ctx* c, const uint8_t* rgba8, int n) {
   c->tfst_dirty = true;
   int rc = ensure(c, &c->d_tf1d, &c->tf1d_cap, 4 * (size_t)n);
   if (!rc) rc = ensure(c, &c->d_tf1f, &c->tf1f_cap, (size_t)n);
+  if (!rc) rc = ensure(c, &c->d_tf1next, &c->tf1next_cap, (size_t)n);
   if (rc) return rc;
+  std::vector<uint16_t> next((size_t)n);
+  for (int i = n - 1; i >= 0; --i)
+    next[(size_t)i] = rgba8[4 * (size_t)i + 3] ? (uint16_t)i : (i + 1 < n ? next[(size_t)i + 1] : (uint16_t)0xffff);
   // texture1D of the RGBA8 table returns byte/255 (GL_NEAREST): expand once
   const std::vector<float4> f = unorm_table(rgba8, (size_t)n);
   HIPCHK(c, hipMemcpyAsync(c->d_tf1d, c->tf1d.data(), 4 * (size_t)n, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->d_tf1f, f.data(), f.size() * sizeof(float4), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, hipMemcpyAsync(c->d_tf1next, next.data(), next.size() * sizeof(uint16_t), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return TVK_OK;
 }
@@ -1123,51 +1140,61 @@ int learn_prepare(tvk_ctx* c) {
   return ensure_cells(c);
 }
 
+int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads) {
+  const Layout& L = c->L;
+  std::vector<GatherBrick> gb(L.toc.size());
+  std::vector<uint32_t> base(L.toc.size(), 0);
+  uint64_t total = 0;
+  uint32_t max_cells = 0, max_vox = 0;
+  for (size_t i = 0; i < L.toc.size(); ++i) {
+    for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)L.toc[i].coords[k]; gb[i].n[k] = L.toc[i].size[k]; }
+    gb[i].offset = L.toc[i].offset;
+    const uint32_t nc = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
+    base[i] = (uint32_t)total;
+    total += nc;
+    max_cells = std::max(max_cells, nc);
+    max_vox = std::max(max_vox, (uint32_t)L.toc[i].count);
+  }
+  if (total >= (1ull << 32)) return fail(c, TVK_ERR_UNSUPPORTED, "cell grid exceeds 2^32 cells");
+  std::shared_ptr<void> gb_hold, base_hold, quad_hold;
+  hipError_t e = hipSuccess;
+  if (!G.hold) e = device_block(&G.hold, std::max<uint64_t>(total, 1) * sizeof(uint32_t));
+  if (e == hipSuccess) e = device_block(&gb_hold, gb.size() * sizeof(GatherBrick));
+  if (e == hipSuccess) e = device_block(&base_hold, base.size() * sizeof(uint32_t));
+  if (e == hipSuccess && !quads) e = device_block(&quad_hold, quad_words(L) * sizeof(uint32_t));
+  if (e != hipSuccess) return hipfail(c, "cell grid", e);
+  GatherBrick* const d_gb = (GatherBrick*)gb_hold.get();
+  e = hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(base_hold.get(), base.data(), base.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess && !quads) {
+    e = launch_minmax(c->d_pool, L.bpv, d_gb, (uint32_t)gb.size(), max_vox, nullptr, (uint32_t*)quad_hold.get(), c->stream);
+    quads = (const uint32_t*)quad_hold.get();
+  }
+  if (e == hipSuccess)
+    e = launch_cells(quads, L.bpv, d_gb, (const uint32_t*)base_hold.get(), (uint32_t)gb.size(), max_cells,
+                     (uint32_t*)G.hold.get(), c->stream);
+  const hipError_t se = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = se;
+  if (e != hipSuccess) return hipfail(c, "cell grid", e);
+  G.d = (uint32_t*)G.hold.get();
+  G.base = std::move(base);
+  G.ready.store(true, std::memory_order_release);
+  return TVK_OK;
+}
+
 int ensure_cells(tvk_ctx* c) {
   if (budgeted(c)) return fail(c, TVK_ERR_UNSUPPORTED, "the cell grid needs every brick resident (pool budget 0)");
   if (c->ingest_pending) return fail(c, TVK_ERR_STATE, "not every brick was uploaded");
   if (!c->cells) return fail(c, TVK_ERR_STATE, "no dataset");
   CellGrid& G = *c->cells;
-  if (G.d) return TVK_OK;
-  const Layout& L = c->L;
-  std::vector<GatherBrick> gb(L.toc.size());
-  G.base.assign(L.toc.size(), 0);
-  uint64_t total = 0;
-  uint32_t max_cells = 0;
-  for (size_t i = 0; i < L.toc.size(); ++i) {
-    for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)L.toc[i].coords[k]; gb[i].n[k] = L.toc[i].size[k]; }
-    gb[i].offset = L.toc[i].offset;
-    const uint32_t nc = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
-    G.base[i] = (uint32_t)total;
-    total += nc;
-    max_cells = std::max(max_cells, nc);
-  }
-  if (total >= (1ull << 32)) return fail(c, TVK_ERR_UNSUPPORTED, "cell grid exceeds 2^32 cells");
-  GatherBrick* d_gb = nullptr;
-  uint32_t* d_base = nullptr;
-  uint32_t* d_cells = nullptr;
-  hipError_t e = device_alloc(&d_cells, std::max<uint64_t>(total, 1) * sizeof(uint32_t));
-  if (e == hipSuccess) e = device_alloc(&d_gb, gb.size() * sizeof(GatherBrick));
-  if (e == hipSuccess) e = device_alloc(&d_base, G.base.size() * sizeof(uint32_t));
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(d_base, G.base.data(), G.base.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) e = launch_cells(c->d_pool, L.bpv, d_gb, d_base, (uint32_t)gb.size(), max_cells, d_cells, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  if (d_gb) (void)hipFree(d_gb);
-  if (d_base) (void)hipFree(d_base);
-  if (e != hipSuccess) {
-    if (d_cells) (void)hipFree(d_cells);
-    return hipfail(c, "cell grid", e);
-  }
-  G.d = d_cells;
-  return TVK_OK;
+  if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
+  std::lock_guard<std::mutex> lk(G.mu);
+  return G.ready.load(std::memory_order_acquire) ? TVK_OK : make_cells(c, G, nullptr);
 }
 
 void brick_tf_stats(tvk_ctx* c, FrameBrick& fb) {
   const tvk_ctx::TfStats& T = c->tfst;
-  fb.cells = c->cells && !c->cells->base.empty() ? c->cells->base[fb.toc] : 0u;
   for (float& v : fb.tfs) v = 0.0f;
   if (T.n <= 0 || c->P.mode == TVK_RM_ISOSURFACE) return;
   // TF coordinate and entry of a stored value, as the march computes them
@@ -1195,6 +1222,7 @@ void fill_shade(const tvk_ctx* c, ShadeConst& S) {
   S.tf1 = c->d_tf1f;
   S.tf2f = c->d_tf2f;
   S.tf2_cols = c->d_tf2cols;
+  S.tf1_next = c->d_tf1next;
   S.tf_n = c->tf1d_n;
   S.tf_w = c->tf2d_w;
   S.tf_h = c->tf2d_h;
@@ -1215,14 +1243,14 @@ void fill_shade(const tvk_ctx* c, ShadeConst& S) {
   S.tfst = c->d_tfst;
   S.tfst_n = c->tfst.n;
   S.tfst_levels = c->tfst.levels;
-  S.cells = c->cells ? c->cells->d : nullptr;
+  S.cells = cells_device(c);
   S.overlap = (int)c->L.overlap;
 }
 
 // The launch of an allocation-free render: the planned lists go to the
 // caller's buffers (fixed), checked against their capacities.
 static int launch_fixed(tvk_ctx* c, int nviews, uint64_t pixels, uint32_t groups, uint32_t in_list,
-                        const FrameBuffers& fx, tvk_stats* st) {
+                        const FrameBuffers& fx, const uint32_t* cells, tvk_stats* st) {
   if (c->h_list.size() > fx.list_cap)
     return fail(c, TVK_ERR_ARG, "visible-brick list (" + std::to_string(c->h_list.size()) +
                                     " entries) exceeds the allocation-free render's limit of " +
@@ -1238,6 +1266,7 @@ static int launch_fixed(tvk_ctx* c, int nviews, uint64_t pixels, uint32_t groups
                            c->stream));
   MarchArgs a{};
   fill_shade(c, a.S);
+  a.S.cells = cells;
   a.list = fx.list;
   a.views = fx.views;
   a.mode = c->P.mode;
@@ -1306,6 +1335,7 @@ int render_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_
     int rc = learn_prepare(c);
     if (rc) return rc;
   }
+  const uint32_t* const cells = fixed ? cells_device(c) : cells_for_render(c);
   c->h_list.clear();
   c->h_views.assign((size_t)nviews, ViewConst{});
   std::vector<PlannedBrick> planned;
@@ -1327,6 +1357,7 @@ int render_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_
     vc.list_offset = (uint32_t)c->h_list.size();
     make_frame_bricks(c->L, V, pp, planned, c->h_list, compat_dims(c), compat_offsets(c));
     vc.nlist = (uint32_t)c->h_list.size() - vc.list_offset;
+    brick_cells(c, cells, c->h_list.data() + vc.list_offset, vc.nlist);
     if (learn > 0)
       for (size_t q = vc.list_offset; q < c->h_list.size(); ++q) brick_tf_stats(c, c->h_list[q]);
     vc.out_offset = (uint32_t)pixels;
@@ -1336,7 +1367,7 @@ int render_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_
     c->last_lod = lod;
   }
   if (pixels >= (1ull << 32)) return fail(c, TVK_ERR_ARG, "too many pixels in one call");
-  if (fixed) return launch_fixed(c, nviews, pixels, groups, in_list, *fixed, st);
+  if (fixed) return launch_fixed(c, nviews, pixels, groups, in_list, *fixed, cells, st);
   // the dispatch order (raster: none)
   const int dorder = c->dispatch & 3;
   const bool ordered = dorder != TVK_DISPATCH_RASTER && groups > 0;
@@ -1373,6 +1404,7 @@ int render_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_
                              c->stream));
   MarchArgs a{};
   fill_shade(c, a.S);
+  a.S.cells = cells;
   a.list = c->d_list;
   a.views = c->d_views;
   a.mode = c->P.mode;

@@ -128,6 +128,7 @@ int plan_batch(tvk_batch* b, uint32_t* bricks_total) {
     bool lit;
     int bpv;
     uint32_t ntoc;
+    const uint32_t* cells;
     std::vector<FrameBrick> list;
   };
   std::vector<Planned> P(b->reqs.size());
@@ -166,6 +167,8 @@ int plan_batch(tvk_batch* b, uint32_t* bricks_total) {
       if (!rc) {
         plan_frame(c->L, c->minmax, c->range_max, V, pp, planned);
         make_frame_bricks(c->L, V, pp, planned, P[i].list, compat_dims(c), compat_offsets(c));
+        P[i].cells = cells_for_render(c);
+        brick_cells(c, P[i].cells, P[i].list.data(), P[i].list.size());
         if (b->net && c->P.mode != TVK_RM_ISOSURFACE) {
           rc = learn_prepare(c);
           if (!rc)
@@ -177,6 +180,7 @@ int plan_batch(tvk_batch* b, uint32_t* bricks_total) {
     BatchRequest& br = P[i].br;
     br = BatchRequest{};
     fill_shade(c, br.S);
+    br.S.cells = P[i].cells;
     make_view_const(V, br.V);
     br.V.nlist = (uint32_t)P[i].list.size();
     br.V.out_offset = (uint32_t)pixels;

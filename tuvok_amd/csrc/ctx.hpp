@@ -6,7 +6,9 @@
 #include <cstdio>
 #include <cstring>
 #include <limits>
+#include <atomic>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -21,14 +23,14 @@ hipError_t launch_march(const MarchArgs& a, int bpv, hipStream_t st, int learn);
 hipError_t launch_batch(const BatchArgs& b, int mode, bool lit, int bpv, int groups, hipStream_t st, int learn);
 hipError_t launch_gather(const void* lin, int bpv, const uint64_t dims[3], const GatherBrick* d_bricks, uint32_t nb,
                          uint32_t row_len, uint32_t max_vox, void* pool, const uint32_t core[3], uint32_t ov, int clamp,
-                         uint32_t* mm, hipStream_t st);
+                         uint32_t* mm, uint32_t* quads, hipStream_t st);
 hipError_t launch_downsample(const void* src, const uint64_t sd[3], void* dst, const uint64_t dd[3], int bpv,
                              hipStream_t st, int median);
 hipError_t launch_downsample_bricks(void* pool, int bpv, const GatherBrick* d_coarse, uint32_t nb,
                                     const GatherBrick* d_fine, const uint32_t fine_bricks[3], uint32_t ov,
                                     const uint32_t split[3], uint64_t max_elems, int median, hipStream_t st);
 hipError_t launch_minmax(const void* pool, int bpv, const GatherBrick* d_bricks, uint32_t nb, uint32_t max_vox,
-                         uint32_t* out, hipStream_t st);
+                         uint32_t* out, uint32_t* quads, hipStream_t st);
 hipError_t launch_unswizzle(const void* pool, int bpv, const GatherBrick* d_bricks, const uint64_t* d_ref_off,
                             uint32_t nb, uint32_t max_vox, void* out, hipStream_t st);
 hipError_t launch_max_gradient(const void* lin, int bpv, const uint64_t d[3], int clamp, double* out, uint32_t blocks,
@@ -44,7 +46,7 @@ hipError_t launch_extend(void* pool, int bpv, const GatherBrick* d_bricks, uint3
                          hipStream_t st);
 hipError_t launch_display(const float* frames, uint32_t W, uint32_t H, uint32_t nviews, const float top[3],
                           const float bottom[3], uint8_t* out, hipStream_t st);
-hipError_t launch_cells(const void* pool, int bpv, const GatherBrick* d_bricks, const uint32_t* d_base, uint32_t nb,
+hipError_t launch_cells(const uint32_t* quads, int bpv, const GatherBrick* d_bricks, const uint32_t* d_base, uint32_t nb,
                         uint32_t max_cells, uint32_t* out, hipStream_t st);
 hipError_t launch_brick_max_gradient(const void* pool, int bpv, const GatherBrick* d_bricks, uint32_t nb,
                                      uint32_t ov, uint32_t gx, double* out, hipStream_t st);
@@ -90,13 +92,17 @@ struct PoolState {
   ~PoolState();
 };
 
-// Cell grid of a dataset (learned mode): per brick, the (min, max) of its cells
-// (tvk_types.hpp), built on first use and shared by the contexts that share
-// the dataset.
+// Cell grid of a dataset: per brick, the (min, max) of its cells (tvk_types.hpp),
+// from which the march knows the stretches of a ray that cannot contribute.  Made
+// with the bricks, or on first use for bricks handed over one by one; shared by
+// the contexts that share the dataset.  A brick uploaded again clears `ready` for
+// all of them; the next use makes the words again in place.
 struct CellGrid {
+  std::mutex mu;                // held while it is made
+  std::atomic<bool> ready{false};
+  std::shared_ptr<void> hold;
   uint32_t* d = nullptr;
   std::vector<uint32_t> base;   // first cell of each TOC brick
-  ~CellGrid() { if (d) (void)hipFree(d); }
 };
 }  // namespace tvk
 
@@ -138,7 +144,8 @@ struct tvk_ctx {
   float4* d_tf2f = nullptr;
   float build_ms = 0.0f;         // device time of the last bricking (build_pool)
   uint64_t* d_tf2cols = nullptr;  // 64 words: value columns of the 2D TF with a non-zero alpha
-  size_t tf1d_cap = 0, tf2d_cap = 0, tf1f_cap = 0, tf2f_cap = 0;
+  uint16_t* d_tf1next = nullptr;  // per 1D TF entry: the first one from it on with a non-zero alpha
+  size_t tf1d_cap = 0, tf2d_cap = 0, tf1f_cap = 0, tf2f_cap = 0, tf1next_cap = 0;
   // view + parameters
   ViewState V;
   bool has_view = false;
@@ -293,12 +300,21 @@ int frame_lod(tvk_ctx* c, const ViewState& V, int* lod);
 int plan_params(tvk_ctx* c, int lod, PlanParams& pp);
 // GLRenderer::CalculateScaling
 float tf_scale_of(const tvk_ctx* c);
-// TF statistics over a brick's value range (FrameBrick::tfs) and its cell grid
+// TF statistics over a brick's value range (FrameBrick::tfs)
 void brick_tf_stats(tvk_ctx* c, FrameBrick& fb);
 // learned mode: device TF statistics of the active TF and the dataset's cell grid
 int learn_prepare(tvk_ctx* c);
-// the dataset's cell grid (built on first use)
+// the dataset's cell grid (made on first use)
 int ensure_cells(tvk_ctx* c);
+// The cell grid from quad ranges of every brick (quads, or null: read from the
+// pool), stream-ordered; needs G.mu.
+int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads);
+inline size_t quad_words(const Layout& L) { return (size_t)(L.pool_elems / (L.bpv == 1 ? 256u : 128u)) * (L.bpv == 1 ? 2u : 1u); }
+// the cell grid as the kernels read it; null while it is not made, for
+// compatibility textures and for a budgeted pool
+inline const uint32_t* cells_device(const tvk_ctx* c) {
+  return !compat_active(c) && !c->pst && c->cells && c->cells->ready.load(std::memory_order_acquire) ? c->cells->d : nullptr;
+}
 // the step network as the kernels read it (false when s is null)
 bool stepnet_device(const struct tvk_stepnet* s, StepNetDev* out);
 // shading constants of the context's dataset, TF and parameters
@@ -317,6 +333,19 @@ int pool_set_budget(tvk_ctx* c, uint64_t budget_bytes);
 // Copies bricks [first, first+n) in the reference layout to host memory.
 int pool_download(tvk_ctx* c, size_t first, size_t n, void* host, size_t bytes);
 inline bool budgeted(const tvk_ctx* c) { return c->pst != nullptr; }
+// first cells of the listed bricks (cells: cells_device's, may be null)
+inline void brick_cells(const tvk_ctx* c, const uint32_t* cells, FrameBrick* fb, size_t n) {
+  for (size_t i = 0; i < n; ++i) fb[i].cells = cells ? c->cells->base[fb[i].toc] : 0u;
+}
+// The cell grid for a render of the context, made if that has not happened; null
+// where the bricks have none (a march without it samples every step).
+inline const uint32_t* cells_for_render(tvk_ctx* c) {
+  if (!budgeted(c) && !compat_active(c) && c->cells && !c->cells->ready.load(std::memory_order_acquire)) {
+    const std::string msg = c->err;
+    if (ensure_cells(c) != TVK_OK) { (void)hipGetLastError(); c->err = msg; }
+  }
+  return cells_device(c);
+}
 // a frame of a budgeted dataset (fixed step, any mode)
 int render_budget_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_stats* st);
 

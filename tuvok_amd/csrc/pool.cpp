@@ -629,7 +629,7 @@ int tvk_upload_brick(tvk_ctx* c, uint32_t lod, uint64_t index, const void* data,
     --c->ingest_pending;
   }
   c->cp = tvk_ctx::CompatPool{};   // made again from the new contents on the next render
-  if (c->cells && c->cells->d) c->cells = std::make_shared<CellGrid>();   // rebuilt on next use
+  if (c->cells) c->cells->ready.store(false, std::memory_order_release);   // made again on next use
   return TVK_OK;
 }
 

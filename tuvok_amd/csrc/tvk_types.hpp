@@ -43,7 +43,7 @@ struct FrameBrick {
   uint64_t offset;      // element offset of the brick in the pool
   int16_t rect[4];      // conservative pixel rectangle x0,y0,x1,y1 (inclusive)
   uint32_t toc;         // TOC index of the brick
-  uint32_t cells;       // first entry of the brick's cell grid (learned mode)
+  uint32_t cells;       // first entry of the brick's cell grid (ShadeConst::cells)
   // transfer-function statistics over the brick's value range (step proposal
   // features): vmin, vmax (TF coordinates), alpha mean, alpha max, alpha total
   // variation, colour total variation, largest alpha step, fraction of the
@@ -84,14 +84,13 @@ struct ShadeConst {
   const float4* tf1;            // 1D TF as float4 (byte / 255), tf_n entries
   const float4* tf2f;           // 2D TF as float4 (byte / 255), tf_w x tf_h
   const uint64_t* tf2_cols;     // bit x: value column x of the 2D TF has a non-zero alpha (64 words)
+  const uint16_t* tf1_next;     // per 1D TF entry: the first entry from it on with a non-zero alpha (0xffff: none)
   int tf_n, tf_w, tf_h;
   float tf_scale, grad_scale, iso_n, ert_eps;
   float dscale[3], amb[3], dif[3], spc[3], ldir[3], iso_col[3];
   int refine_steps, clamp_edge;
-  // learned mode: per-entry TF statistics (layout of tf_stats_layout) and the
-  // dataset's cell grid (cell_grid_dims)
-  const float* tfst;
-  const uint32_t* cells;
+  const float* tfst;            // learned mode: per-entry TF statistics (layout of tf_stats_layout)
+  const uint32_t* cells;        // the dataset's cell grid (null: none for these bricks)
   int tfst_n, tfst_levels;
   int overlap;                  // brick overlap of the dataset
 };
