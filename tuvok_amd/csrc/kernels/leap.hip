@@ -411,12 +411,44 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
           int steps = (int)ceilf(length(pout - pin) / stepSize);
           steps = min(steps, (int)ceilf(length((exitN - cur) * sc) / stepSize));
           V3 b = pin;
-          for (int i = 0; i < steps; ++i) {
+          // The steps whose 4x4x4 neighbourhood lies inside the brick, one range
+          // per segment (the raycaster's rule and margin: each addition of a
+          // position below n rounds by at most n 2^-24, so after i < steps of
+          // them the drift is below steps n 2^-24 voxels).  Every lane takes its
+          // steps before the range, in it and after it as three loops, so only
+          // the few steps next to a brick face pay for per-tap gathers; decided
+          // by one ballot per step, a wave gathered whenever any of its 64 rays
+          // was next to a face.
+          int in_lo = 0, in_hi = -1;
+          if constexpr (LIT || MODE == 1) {
+            float lo = 0.0f, hi = (float)(steps - 1);
+            const float pc[3] = {pin.x, pin.y, pin.z}, sp[3] = {step.x, step.y, step.z};
+            const int nn3[3] = {nx, ny, nz};
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+              const float na = (float)nn3[a], u0 = pc[a] - 0.5f, du = sp[a];
+              const float margin = 0.0625f + (float)steps * na * 0x1p-23f;
+              const float ulo = 1.0f + margin, uhi = na - 2.0f - margin;   // floor(u) in [1, n - 3]
+              if (!(ulo <= uhi) || !(fabsf(u0) < 0x1p24f) || !(fabsf(du) < 0x1p24f)) {
+                hi = -1.0f;
+              } else if (du == 0.0f) {
+                if (!(u0 >= ulo && u0 <= uhi)) hi = -1.0f;
+              } else {
+                const float t1 = (ulo - u0) / du, t2 = (uhi - u0) / du;
+                lo = fmaxf(lo, fminf(t1, t2));
+                hi = fminf(hi, fmaxf(t1, t2));
+              }
+            }
+            if (hi >= lo) { in_lo = (int)ceilf(lo); in_hi = (int)floorf(hi); }
+          }
+          int i = 0;
+          for (int part = 0; part < 3 && !done; ++part) {
+          const int end = part == 0 ? (in_hi >= in_lo ? min(in_lo, steps) : steps) : (part == 1 ? min(in_hi + 1, steps) : steps);
+          for (; i < end; ++i) {
             ++ns;
-            // value (and, for gradients, the cross) from the 32-voxel cross when
-            // every active lane's neighbourhood lies inside its brick
+            // value (and, for gradients, the cross) from the 32-voxel cross
             LeapCross<T> X;
-            const bool cross = MODE != 2 && (LIT || MODE == 1) && __ballot(!X.coords(nx, ny, nz, b)) == 0;
+            const bool cross = MODE != 2 && (LIT || MODE == 1) && part == 1 && __ballot(!X.coords(nx, ny, nz, b)) == 0;
             const float data = cross ? X.value(bd, nx, ny) : sample_vox_fast<T>(bd, nx, ny, nz, b);
             auto grad = [&]() { return cross ? X.gradient() : gradient_vox<T>(bd, nx, ny, nz, b); };
             if constexpr (MODE == 2) {
@@ -481,6 +513,7 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
             if (acc[3] > 0.99f) { done = true; break; }
             b = b + step;
           }
+          }
           if (!done) cur = (b - tr) / sc;
         } else {
           cur = bexit + direction * voxelSize / rayLength;
@@ -524,6 +557,10 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
   }
   A.resume[2 * pix] = rpos;
   A.resume[2 * pix + 1] = rcol;
+  // rays to resume (a later pass, or a hit of the isosurface), one atomic per wave
+  const uint64_t open = __ballot(rpos.w != 1000.0f);
+  if (open != 0 && lane == __ffsll((unsigned long long)__ballot(true)) - 1)
+    atomicAdd(A.unfinished, (unsigned int)__popcll(open));
   if (A.counter && ns) atomicAdd(A.counter, (unsigned long long)ns);
 }
 

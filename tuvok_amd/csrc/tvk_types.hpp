@@ -223,6 +223,7 @@ struct LeapArgs {
   const GatherBrick* bricks;   // per TOC brick: stored size and pool offset
   uint32_t* table;             // GLHashTable of the requested bricks: serialised 4D brick index + 1, 0 = free
   uint32_t table_size, rehash; // entries; probes per request (GLHashTable.cpp:140-181)
+  unsigned int* unfinished;    // counts the pass's rays whose resume w is not 1000 (cleared before the launch)
   float4* resume;              // 2 per pixel: (normalised position, eye z; w = 1000 finished), colour
   float* out;                  // RGBA32F accumulated colour
   unsigned long long* counter; // samples (or nullptr)
