@@ -105,7 +105,7 @@ __device__ __forceinline__ float sample_vox_fast(const T* __restrict__ d, int nx
 template <typename T>
 struct LeapCross {
   int ic[3];
-  float fc[3], fm[3], fq[3];
+  float fc[3], fq[3];   // weights of the centre (and the lower taps) and of the upper taps
   float c[2][2][2], xl[2][2], xr[2][2];   // scaled taps, [x][y][z] / [y][z]
   const uint8_t* base;
   uint32_t nbx, nbxy;
@@ -116,15 +116,13 @@ struct LeapCross {
     bool ok = true;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      float s = fminf(fmaxf(bc[a], 0.0f), (float)n[a]), u = s - 0.5f, fl = floorf(u);
+      // b >= 1.5 here (ok), so b - 1 and b - 0.5 are exact: the lower tap has the
+      // centre's weight.  b + 1 rounds where it passes a power of two.
+      const float u = bc[a] - 0.5f, fl = floorf(u);
       ic[a] = (int)fl; fc[a] = u - fl;
-      s = fminf(fmaxf(bc[a] + -1.0f, 0.0f), (float)n[a]); u = s - 0.5f; fl = floorf(u);
-      const int im = (int)fl;
-      fm[a] = u - fl;
-      s = fminf(fmaxf(bc[a] + 1.0f, 0.0f), (float)n[a]); u = s - 0.5f; fl = floorf(u);
-      const int iq = (int)fl;
-      fq[a] = u - fl;
-      ok = ok && ic[a] >= 1 && ic[a] + 2 < n[a] && im == ic[a] - 1 && iq == ic[a] + 1;
+      const float uq = (bc[a] + 1.0f) - 0.5f, fl1 = floorf(uq);
+      fq[a] = uq - fl1;
+      ok = ok && ic[a] >= 1 && ic[a] < n[a] - 2 && (int)fl1 == ic[a] + 1;
     }
     return ok;
   }
@@ -174,15 +172,15 @@ struct LeapCross {
     const float xp = leap_tri(c[1][0][0], xr[0][0], c[1][1][0], xr[1][0], c[1][0][1], xr[0][1], c[1][1][1], xr[1][1],
                               fq[0], fc[1], fc[2]);
     const float xm = leap_tri(xl[0][0], c[0][0][0], xl[1][0], c[0][1][0], xl[0][1], c[0][0][1], xl[1][1], c[0][1][1],
-                              fm[0], fc[1], fc[2]);
+                              fc[0], fc[1], fc[2]);
     const float yp = leap_tri(yl[0][0], yl[1][0], c[0][0][0], c[1][0][0], yl[0][1], yl[1][1], c[0][0][1], c[1][0][1],
-                              fc[0], fm[1], fc[2]);
+                              fc[0], fc[1], fc[2]);
     const float ym = leap_tri(c[0][1][0], c[1][1][0], yr[0][0], yr[1][0], c[0][1][1], c[1][1][1], yr[0][1], yr[1][1],
                               fc[0], fq[1], fc[2]);
     const float zp = leap_tri(c[0][0][1], c[1][0][1], c[0][1][1], c[1][1][1], zr[0][0], zr[1][0], zr[0][1], zr[1][1],
                               fc[0], fc[1], fq[2]);
     const float zm = leap_tri(zl[0][0], zl[1][0], zl[0][1], zl[1][1], c[0][0][0], c[1][0][0], c[0][1][0], c[1][1][0],
-                              fc[0], fc[1], fm[2]);
+                              fc[0], fc[1], fc[2]);
     return mk(xm - xp, yp - ym, zm - zp) / 2.0f;
   }
 };
@@ -199,10 +197,38 @@ __device__ __forceinline__ V3 gradient_vox(const T* __restrict__ d, int nx, int 
   return mk(xm - xp, yp - ym, zm - zp) / 2.0f;
 }
 
+// Shading directions without the compiler's division and square root sequences
+// (about 11 and 15 instructions each; a lit sample had eight and three of them,
+// 130 of its 640 instructions):
+// rsqrt_refined: 1 / sqrt(x) by the hardware estimate and one Newton step, within
+// 0.6 ulp for normal x, where 1 / sqrtf(x) rounds twice; the same values at 0
+// and beyond the normal range decide nothing but an unlit direction.
+__device__ __forceinline__ float rsqrt_refined(float x) {
+  const float r = __builtin_amdgcn_rsqf(x);
+  return fmaf(0.5f * r, fmaf(-(x * r), r, 1.0f), r);
+}
+// a / b from r, b's reciprocal within an ulp: the product moved by its residual,
+// the correctly rounded quotient as division gives it (a and b of ordinary size)
+__device__ __forceinline__ float quotient(float a, float b, float r) {
+  const float q = a * r;
+  return fmaf(fmaf(-q, b, a), r, q);
+}
+__device__ __forceinline__ V3 unit(V3 a) {
+  const float d = dot(a, a);
+  if (__builtin_expect(d < 0x1p-96f, 0)) return normalize(a);
+  return a * rsqrt_refined(d);
+}
+// a / l, l = length(a) > 0
+__device__ __forceinline__ V3 over_length(V3 a, float l) {
+  if (__builtin_expect(l < 0x1p-48f, 0)) return a / l;
+  const float r = rsqrt_refined(dot(a, a));
+  return mk(quotient(a.x, l, r), quotient(a.y, l, r), quotient(a.z, l, r));
+}
+
 // lighting.glsl:33-42 with the model-space eye
 __device__ __forceinline__ V3 lighting_eye(V3 eye, V3 pos, V3 n, V3 amb, V3 dif, V3 spc, V3 L) {
-  const V3 view = normalize(eye - pos);
-  const V3 R = normalize(reflect(view, n));
+  const V3 view = unit(eye - pos);
+  const V3 R = unit(reflect(view, n));
   const float dd = fmaxf(fabsf(dot(n, L)), 0.0f);
   const float ss = pow8(fmaxf(dot(R, L), 0.0f));
   const V3 c = amb + dif * dd + spc * ss;
@@ -259,8 +285,9 @@ __device__ __forceinline__ uint32_t compute_lod(const LeapArgs& A, float depth) 
   return min((uint32_t)(A.nlod - 1), lod);
 }
 
+// cols: the 2D TF's column mask (64 words, MODE 1) in LDS
 template <int MODE, bool LIT, typename T>
-__device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int lane) {
+__device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int lane, const uint64_t* cols) {
   const int tx = (int)(tile % A.tiles_x), ty = (int)(tile / A.tiles_x);
   const int px = tx * 8 + (lane & 7), py = ty * 8 + (lane >> 3);
   if (px >= A.W || py >= A.H) return;   // no wave-level operations below
@@ -411,6 +438,12 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
           int steps = (int)ceilf(length(pout - pin) / stepSize);
           steps = min(steps, (int)ceilf(length((exitN - cur) * sc) / stepSize));
           V3 b = pin;
+          // (b - tr) / sc of a shaded sample
+          const V3 rsc = mk(1.0f / sc.x, 1.0f / sc.y, 1.0f / sc.z);
+          auto at = [&](V3 p) {
+            const V3 q = p - tr;
+            return mk(quotient(q.x, sc.x, rsc.x), quotient(q.y, sc.y, rsc.y), quotient(q.z, sc.z, rsc.z));
+          };
           // The steps whose 4x4x4 neighbourhood lies inside the brick, one range
           // per segment (the raycaster's rule and margin: each addition of a
           // position below n rounds by at most n 2^-24, so after i < steps of
@@ -478,28 +511,28 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
               c[0] = tv.x; c[1] = tv.y; c[2] = tv.z; c[3] = tv.w;
               if (LIT) {
                 V3 g = grad() * dsc;
-                const float l = length(g);
-                if (l > 0.0f) g = mk(g.x / l, g.y / l, g.z / l);
-                const V3 lc = lighting_eye(meye, (b - tr) / sc, g, amb, mk(c[0], c[1], c[2]) * dif, spc, mlight);
+                const float l = sqrt_rn(dot(g, g));
+                if (l > 0.0f) g = over_length(g, l);
+                const V3 lc = lighting_eye(meye, at(b), g, amb, mk(c[0], c[1], c[2]) * dif, spc, mlight);
                 c[0] = lc.x; c[1] = lc.y; c[2] = lc.z;
               }
             } else {
               const float sx = fminf(fmaxf(data * S.tf_scale, 0.0f), 1.0f);
               const int xi = min((int)floorf(sx * (float)S.tf_w), S.tf_w - 1);
-              if (((S.tf2_cols[xi >> 6] >> (xi & 63)) & 1ull) == 0) {
+              if (((cols[xi >> 6] >> (xi & 63)) & 1ull) == 0) {
                 // every row of this value column is transparent: alpha 0 whatever
                 // the gradient, so the sample composites to nothing
                 c[0] = c[1] = c[2] = c[3] = 0.0f;
               } else {
                 const V3 g = grad();
-                const float gm = length(g);
+                const float gm = sqrt_rn(dot(g, g));   // length(g), bit for bit
                 const float sy = fminf(fmaxf(1.0f - gm * S.grad_scale, 0.0f), 1.0f);
                 const int yi = min((int)floorf(sy * (float)S.tf_h), S.tf_h - 1);
                 const float4 tv = S.tf2f[(size_t)yi * (size_t)S.tf_w + (size_t)xi];
                 c[0] = tv.x; c[1] = tv.y; c[2] = tv.z; c[3] = tv.w;
                 if (LIT) {
-                  const V3 nrm = dsc * (gm > 0.0f ? g / gm : g);
-                  const V3 lc = lighting_eye(meye, (b - tr) / sc, nrm, amb, mk(c[0], c[1], c[2]) * dif, spc, mlight);
+                  const V3 nrm = dsc * (gm > 0.0f ? over_length(g, gm) : g);
+                  const V3 lc = lighting_eye(meye, at(b), nrm, amb, mk(c[0], c[1], c[2]) * dif, spc, mlight);
                   c[0] = lc.x; c[1] = lc.y; c[2] = lc.z;
                 }
               }
@@ -568,9 +601,14 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
 // then from the others' (pull_tiles)
 template <int MODE, bool LIT, typename T>
 __global__ __launch_bounds__(256) void leap_kernel(LeapArgs A) {
+  __shared__ uint64_t s_cols[MODE == 1 ? 64 : 1];
   const int lane = threadIdx.x & 63;
+  if constexpr (MODE == 1) {
+    if (threadIdx.x < 64) s_cols[threadIdx.x] = A.S.tf2_cols[threadIdx.x];
+    __syncthreads();   // the only workgroup barrier
+  }
   pull_tiles(A.queues, A.xcd_items,
-             [&](uint32_t x, uint32_t t) { leap_tile<MODE, LIT, T>(A, x * A.xcd_items[0] + t, lane); });
+             [&](uint32_t x, uint32_t t) { leap_tile<MODE, LIT, T>(A, x * A.xcd_items[0] + t, lane, s_cols); });
 }
 
 template <int M, bool L, typename T>
