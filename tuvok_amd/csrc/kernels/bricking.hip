@@ -564,8 +564,8 @@ __global__ __launch_bounds__(256) void max_gradient(const T* __restrict__ lin, u
 // squared length of the integer differences is exact (double for 16-bit voxels,
 // 33 bits), so a lane keeps the differences of its largest and forms the
 // magnitude, with the reference's divisions and square root, once at the end
-// instead of six divisions and a root per voxel: bounded by HBM and no longer
-// by double-precision arithmetic (1024^3 uint16, 512 bricks: 9.7 -> 1.0 ms).
+// instead of six divisions and a root per voxel; what is left is the integer and
+// conversion work per voxel, not HBM (1024^3 uint16, 512 bricks: 9.7 -> 2.5 ms).
 template <typename T>
 __global__ __launch_bounds__(256) void brick_max_gradient(const T* __restrict__ pool,
                                                           const GatherBrick* __restrict__ bricks, uint32_t ov,

@@ -39,6 +39,12 @@ struct StepNetDev {
   const float* b3;       // [2]
 };
 
+// The same arrays as the training step writes them.
+struct StepNetPack {
+  uint16_t *w1t, *w2t, *w2, *w3t;
+  float *b1, *b2, *b3;
+};
+
 typedef __bf16 sn_bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short sn_u16x8 __attribute__((ext_vector_type(8)));
 typedef float sn_f32x16 __attribute__((ext_vector_type(16)));

@@ -11,8 +11,9 @@ hipError_t launch_sn_pack(const float* th, uint16_t* w1t, uint16_t* w2t, uint16_
 hipError_t launch_sn_infer(const StepNetDev& N, const float* feat, int n, float* out, hipStream_t st);
 hipError_t launch_sn_grad(const StepNetDev& N, const float* W3f, const float* feat, const float* tgt,
                           const uint32_t* idx, int n, float inv_batch, float* part, float* grad, hipStream_t st);
-hipError_t launch_sn_adam(float* th, float* m, float* v, const float* grad, float lr, float b1, float b2, float eps,
-                          int step, float wd, hipStream_t st);
+hipError_t launch_sn_step(const StepNetDev& N, const StepNetPack& P, float* th, float* m, float* v, const float* feat,
+                          const float* tgt, const uint32_t* idx, int n, float inv_batch, float* part, float lr,
+                          float b1, float b2, float eps, int step, float wd, float* loss, hipStream_t st);
 }  // namespace tvk
 
 struct tvk_stepnet {
@@ -27,6 +28,8 @@ struct tvk_stepnet {
   float* d_b = nullptr;       // b1 | b2 | b3
   float* d_part = nullptr;
   size_t part_cap = 0;
+  float* d_loss = nullptr;    // the losses of an epoch's batches
+  size_t loss_cap = 0;
   // training data
   float* d_feat = nullptr;
   float* d_tgt = nullptr;
@@ -143,7 +146,7 @@ void tvk_stepnet_destroy(tvk_stepnet* s) {
   if (!s) return;
   (void)hipSetDevice(s->device);
   if (s->stream) (void)hipStreamSynchronize(s->stream);
-  for (void* p : {(void*)s->d_theta, (void*)s->d_m, (void*)s->d_v, (void*)s->d_grad, (void*)s->d_w, (void*)s->d_b,
+  for (void* p : {(void*)s->d_loss, (void*)s->d_theta, (void*)s->d_m, (void*)s->d_v, (void*)s->d_grad, (void*)s->d_w, (void*)s->d_b,
                   (void*)s->d_part, (void*)s->d_feat, (void*)s->d_tgt, (void*)s->d_idx, (void*)s->d_io})
     if (p) (void)hipFree(p);
   if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -238,33 +241,34 @@ int tvk_stepnet_train(tvk_stepnet* s, int n, int epochs, int batch, float lr, fl
   const size_t tiles = ((size_t)batch + 63) / 64;
   int rc = sensure(s, &s->d_part, &s->part_cap, tiles * (SN_NPARAM + 1));
   if (rc) return rc;
+  const size_t batches = ((size_t)n + (size_t)batch - 1) / (size_t)batch;
+  rc = sensure(s, &s->d_loss, &s->loss_cap, batches);
+  if (rc) return rc;
+  const StepNetDev N = s->dev();
+  const StepNetPack P{const_cast<uint16_t*>(N.w1t), const_cast<uint16_t*>(N.w2t), const_cast<uint16_t*>(N.w2),
+                      const_cast<uint16_t*>(N.w3t), const_cast<float*>(N.b1), const_cast<float*>(N.b2),
+                      const_cast<float*>(N.b3)};
+  std::vector<float> bl(batches);
   std::vector<uint32_t> perm((size_t)n);
   for (int i = 0; i < n; ++i) perm[(size_t)i] = (uint32_t)i;
   std::mt19937_64 g(seed);
-  std::vector<float> gl(SN_NPARAM + 1);
   for (int ep = 0; ep < epochs; ++ep) {
     std::shuffle(perm.begin(), perm.end(), g);
     SCHK(s, hipMemcpyAsync(s->d_idx, perm.data(), perm.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s->stream));
-    double lsum = 0.0;
-    for (int b0 = 0; b0 < n; b0 += batch) {
+    size_t k = 0;
+    for (int b0 = 0; b0 < n; b0 += batch, ++k) {
       const int nb = std::min(batch, n - b0);
-      SCHK(s, launch_sn_grad(s->dev(), s->d_theta + SN_OFF_W3, s->d_feat, s->d_tgt, s->d_idx + b0, nb,
-                             1.0f / (float)nb, s->d_part, s->d_grad, s->stream));
       ++s->adam_step;
-      SCHK(s, launch_sn_adam(s->d_theta, s->d_m, s->d_v, s->d_grad, lr, 0.9f, 0.999f, 1e-8f, s->adam_step,
-                             weight_decay, s->stream));
-      rc = repack(s);
-      if (rc) return rc;
-      if (losses) {
-        float l = 0.0f;
-        SCHK(s, hipMemcpyAsync(&l, s->d_grad + SN_NPARAM, sizeof(float), hipMemcpyDeviceToHost, s->stream));
-        SCHK(s, hipStreamSynchronize(s->stream));
-        lsum += l;
-      }
+      SCHK(s, launch_sn_step(N, P, s->d_theta, s->d_m, s->d_v, s->d_feat, s->d_tgt, s->d_idx + b0, nb, 1.0f / (float)nb,
+                             s->d_part, lr, 0.9f, 0.999f, 1e-8f, s->adam_step, weight_decay, s->d_loss + k, s->stream));
     }
+    SCHK(s, hipMemcpyAsync(bl.data(), s->d_loss, batches * sizeof(float), hipMemcpyDeviceToHost, s->stream));
+    // the permutation is shuffled and uploaded again for the next epoch
+    SCHK(s, hipStreamSynchronize(s->stream));
+    double lsum = 0.0;
+    for (float l : bl) lsum += l;
     if (losses) losses[ep] = (float)(lsum / n);
   }
-  SCHK(s, hipStreamSynchronize(s->stream));
   return TVK_OK;
 }
 
