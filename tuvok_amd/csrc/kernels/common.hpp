@@ -92,6 +92,25 @@ __device__ __forceinline__ uint32_t oz(int z, uint32_t nbxy) {
   return (((uint32_t)(z >> 2) * nbxy) << (L + 5)) + ((uint32_t)(z & 3) << (L + 3));
 }
 
+// Byte offsets of a footprint's rows in the blocked layout (256-byte blocks, rows
+// 16 bytes apart in y and 64 in z): the row of (y, z) from one product per axis,
+// its neighbours by the step to them, one compare and select each, instead of a
+// shift, a product and two masks per row.  The steps may wrap below 0; sums are
+// modulo 2^32 and end inside the brick.
+struct RowSteps {
+  uint32_t yb, zb;   // bytes from a block to the next in y and z (the same for every lane)
+  __device__ __forceinline__ RowSteps(uint32_t nbx, uint32_t nbxy) : yb(nbx << 8), zb(nbxy << 8) {}
+  __device__ __forceinline__ uint32_t at(int y, int z) const {
+    return (uint32_t)(y >> 2) * yb + (uint32_t)(z >> 2) * zb + ((uint32_t)(y & 3) << 4) + ((uint32_t)(z & 3) << 6);
+  }
+  __device__ __forceinline__ uint32_t ym1(int y) const { return (y & 3) == 0 ? 48u - yb : 0u - 16u; }
+  __device__ __forceinline__ uint32_t yp1(int y) const { return (y & 3) == 3 ? yb - 48u : 16u; }
+  __device__ __forceinline__ uint32_t yp2(int y) const { return (y & 3) >= 2 ? yb - 32u : 32u; }
+  __device__ __forceinline__ uint32_t zm1(int z) const { return (z & 3) == 0 ? 192u - zb : 0u - 64u; }
+  __device__ __forceinline__ uint32_t zp1(int z) const { return (z & 3) == 3 ? zb - 192u : 64u; }
+  __device__ __forceinline__ uint32_t zp2(int z) const { return (z & 3) >= 2 ? zb - 128u : 128u; }
+};
+
 // Runs of voxels along x of the blocked layout.  A row holds its block's W
 // voxels followed by the next block's first W (16 bytes), so voxels s .. s+m-1
 // of a row (s < W, s + m <= 2W) are contiguous.

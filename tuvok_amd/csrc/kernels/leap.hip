@@ -83,13 +83,15 @@ __device__ __forceinline__ float sample_vox_fast(const T* __restrict__ d, int nx
   const float inv = Unorm<T>::inv();
   const uint32_t nbx = nblocks((uint32_t)nx, Blk<T>::LX), nbxy = nbx * nblocks((uint32_t)ny, 2);
   const uint8_t* __restrict__ base = reinterpret_cast<const uint8_t*>(d);
+  const RowSteps R(nbx, nbxy);
+  const uint32_t v00 = R.at(i0[1], i0[2]) + ox<T>(i0[0]) * (uint32_t)sizeof(T), dy = R.yp1(i0[1]), dz = R.zp1(i0[2]);
   float c[2][2][2];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       uint32_t v[2];
-      run2<T>(base, (ox<T>(i0[0]) + oy<T>(i0[1] + j, nbx) + oz<T>(i0[2] + k, nbxy)) * (uint32_t)sizeof(T), v);
+      run2<T>(base, v00 + (j ? dy : 0u) + (k ? dz : 0u), v);
       c[0][j][k] = (float)v[0] * inv;
       c[1][j][k] = (float)v[1] * inv;
     }
@@ -108,7 +110,7 @@ struct LeapCross {
   float fc[3], fq[3];   // weights of the centre (and the lower taps) and of the upper taps
   float c[2][2][2], xl[2][2], xr[2][2];   // scaled taps, [x][y][z] / [y][z]
   const uint8_t* base;
-  uint32_t nbx, nbxy;
+  uint32_t nbx, nbxy, row0;
 
   __device__ __forceinline__ bool coords(int nx, int ny, int nz, V3 b) {
     const int n[3] = {nx, ny, nz};
@@ -126,21 +128,21 @@ struct LeapCross {
     }
     return ok;
   }
-  __device__ __forceinline__ uint32_t vox(int x, int y, int z) const {
-    return (ox<T>(x) + oy<T>(y, nbx) + oz<T>(z, nbxy)) * (uint32_t)sizeof(T);
-  }
   __device__ __forceinline__ float value(const T* __restrict__ d, int nx, int ny) {
     base = reinterpret_cast<const uint8_t*>(d);
     nbx = nblocks((uint32_t)nx, Blk<T>::LX);
     nbxy = nbx * nblocks((uint32_t)ny, 2);
     const float inv = Unorm<T>::inv();
+    const RowSteps R(nbx, nbxy);
+    row0 = R.at(ic[1], ic[2]);
     const int xs = ic[0] - 1;
+    const uint32_t r00 = row0 + ((uint32_t)(xs >> Blk<T>::LX) << 8), dy = R.yp1(ic[1]), dz = R.zp1(ic[2]);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         uint32_t v[4];
-        run4<T>(base, vox(xs & ~((1 << Blk<T>::LX) - 1), ic[1] + j, ic[2] + k), xs & ((1 << Blk<T>::LX) - 1), v);
+        run4<T>(base, r00 + (j ? dy : 0u) + (k ? dz : 0u), xs & ((1 << Blk<T>::LX) - 1), v);
         xl[j][k] = (float)v[0] * inv;
         c[0][j][k] = (float)v[1] * inv;
         c[1][j][k] = (float)v[2] * inv;
@@ -151,37 +153,40 @@ struct LeapCross {
   }
   __device__ __forceinline__ V3 gradient() const {
     const float inv = Unorm<T>::inv();
+    const RowSteps R(nbx, nbxy);
+    const uint32_t v00 = row0 + ox<T>(ic[0]) * (uint32_t)sizeof(T), dy = R.yp1(ic[1]), dz = R.zp1(ic[2]);
+    const uint32_t ym = v00 + R.ym1(ic[1]), yp = v00 + R.yp2(ic[1]), zm = v00 + R.zm1(ic[2]), zp = v00 + R.zp2(ic[2]);
     float yl[2][2], yr[2][2], zl[2][2], zr[2][2];   // [x][z] / [x][y]
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       uint32_t a[2], b[2];
-      run2<T>(base, vox(ic[0], ic[1] - 1, ic[2] + k), a);
-      run2<T>(base, vox(ic[0], ic[1] + 2, ic[2] + k), b);
+      run2<T>(base, ym + (k ? dz : 0u), a);
+      run2<T>(base, yp + (k ? dz : 0u), b);
       yl[0][k] = (float)a[0] * inv; yl[1][k] = (float)a[1] * inv;
       yr[0][k] = (float)b[0] * inv; yr[1][k] = (float)b[1] * inv;
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       uint32_t a[2], b[2];
-      run2<T>(base, vox(ic[0], ic[1] + j, ic[2] - 1), a);
-      run2<T>(base, vox(ic[0], ic[1] + j, ic[2] + 2), b);
+      run2<T>(base, zm + (j ? dy : 0u), a);
+      run2<T>(base, zp + (j ? dy : 0u), b);
       zl[0][j] = (float)a[0] * inv; zl[1][j] = (float)a[1] * inv;
       zr[0][j] = (float)b[0] * inv; zr[1][j] = (float)b[1] * inv;
     }
     // gradient_vox's taps: xp = +x, xm = -x, yp = -y, ym = +y, zp = +z, zm = -z
-    const float xp = leap_tri(c[1][0][0], xr[0][0], c[1][1][0], xr[1][0], c[1][0][1], xr[0][1], c[1][1][1], xr[1][1],
+    const float xpt = leap_tri(c[1][0][0], xr[0][0], c[1][1][0], xr[1][0], c[1][0][1], xr[0][1], c[1][1][1], xr[1][1],
                               fq[0], fc[1], fc[2]);
-    const float xm = leap_tri(xl[0][0], c[0][0][0], xl[1][0], c[0][1][0], xl[0][1], c[0][0][1], xl[1][1], c[0][1][1],
+    const float xmt = leap_tri(xl[0][0], c[0][0][0], xl[1][0], c[0][1][0], xl[0][1], c[0][0][1], xl[1][1], c[0][1][1],
                               fc[0], fc[1], fc[2]);
-    const float yp = leap_tri(yl[0][0], yl[1][0], c[0][0][0], c[1][0][0], yl[0][1], yl[1][1], c[0][0][1], c[1][0][1],
+    const float ypt = leap_tri(yl[0][0], yl[1][0], c[0][0][0], c[1][0][0], yl[0][1], yl[1][1], c[0][0][1], c[1][0][1],
                               fc[0], fc[1], fc[2]);
-    const float ym = leap_tri(c[0][1][0], c[1][1][0], yr[0][0], yr[1][0], c[0][1][1], c[1][1][1], yr[0][1], yr[1][1],
+    const float ymt = leap_tri(c[0][1][0], c[1][1][0], yr[0][0], yr[1][0], c[0][1][1], c[1][1][1], yr[0][1], yr[1][1],
                               fc[0], fq[1], fc[2]);
-    const float zp = leap_tri(c[0][0][1], c[1][0][1], c[0][1][1], c[1][1][1], zr[0][0], zr[1][0], zr[0][1], zr[1][1],
+    const float zpt = leap_tri(c[0][0][1], c[1][0][1], c[0][1][1], c[1][1][1], zr[0][0], zr[1][0], zr[0][1], zr[1][1],
                               fc[0], fc[1], fq[2]);
-    const float zm = leap_tri(zl[0][0], zl[1][0], zl[0][1], zl[1][1], c[0][0][0], c[1][0][0], c[0][1][0], c[1][1][0],
+    const float zmt = leap_tri(zl[0][0], zl[1][0], zl[0][1], zl[1][1], c[0][0][0], c[1][0][0], c[0][1][0], c[1][1][0],
                               fc[0], fc[1], fc[2]);
-    return mk(xm - xp, yp - ym, zm - zp) / 2.0f;
+    return mk(xmt - xpt, ypt - ymt, zmt - zpt) / 2.0f;
   }
 };
 

@@ -267,14 +267,15 @@ __device__ __forceinline__ float sample_brick_iso(const T* __restrict__ d, int n
   if (__ballot(!in) != 0) return sample_brick<T>(d, nx, ny, nz, edge, p);
   const uint32_t nbx = nblocks((uint32_t)nx, Blk<T>::LX), nbxy = nbx * nblocks((uint32_t)ny, 2);
   const uint8_t* __restrict__ b = reinterpret_cast<const uint8_t*>(d);
-  const uint32_t x0 = ox<T>(i0[0]);
+  const RowSteps R(nbx, nbxy);
+  const uint32_t v00 = R.at(i0[1], i0[2]) + ox<T>(i0[0]) * (uint32_t)sizeof(T), dy = R.yp1(i0[1]), dz = R.zp1(i0[2]);
   float c[2][2][2];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       uint32_t v[2];
-      run2<T>(b, (x0 + oy<T>(i0[1] + j, nbx) + oz<T>(i0[2] + k, nbxy)) * (uint32_t)sizeof(T), v);
+      run2<T>(b, v00 + (j ? dy : 0u) + (k ? dz : 0u), v);
       c[0][j][k] = (float)v[0];
       c[1][j][k] = (float)v[1];
     }
@@ -320,15 +321,16 @@ __device__ __forceinline__ void sample_brick_iso_n(const T* __restrict__ d, int 
   }
   const uint32_t nbx = nblocks((uint32_t)nx, Blk<T>::LX), nbxy = nbx * nblocks((uint32_t)ny, 2);
   const uint8_t* __restrict__ b = reinterpret_cast<const uint8_t*>(d);
+  const RowSteps R(nbx, nbxy);
   uint32_t v[N][2][2][2];
 #pragma unroll
   for (int s = 0; s < N; ++s) {
-    const uint32_t x0 = ox<T>(i0[s][0]);
+    const uint32_t v00 = R.at(i0[s][1], i0[s][2]) + ox<T>(i0[s][0]) * (uint32_t)sizeof(T);
+    const uint32_t dy = R.yp1(i0[s][1]), dz = R.zp1(i0[s][2]);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
-        run2<T>(b, (x0 + oy<T>(i0[s][1] + j, nbx) + oz<T>(i0[s][2] + k, nbxy)) * (uint32_t)sizeof(T), v[s][j][k]);
+      for (int k = 0; k < 2; ++k) run2<T>(b, v00 + (j ? dy : 0u) + (k ? dz : 0u), v[s][j][k]);
   }
 #pragma unroll
   for (int s = 0; s < N; ++s) {
@@ -352,28 +354,18 @@ __device__ __forceinline__ void sample_brick_iso_n(const T* __restrict__ d, int 
 // operations are those of the general form.
 template <typename T>
 struct CrossSampler<T, true> {
-  const T* __restrict__ d;
-  int n[3];
-  bool edge;
-  V3 p;
+  const uint8_t* __restrict__ base;
   int ic[3];
   float fc[3];
   float c[2][2][2];
   float xl[2][2], xr[2][2];   // x arms at (y0+j, z0+k)
   uint32_t nbx, nbxy;
+  uint32_t row0;              // byte offset of the row (y0, z0) from the first block column
 
-  // byte offsets of voxel (x, y, z) and of the start of its row
-  __device__ __forceinline__ uint32_t vox(int x, int y, int z) const {
-    return (ox<T>(x) + oy<T>(y, nbx) + oz<T>(z, nbxy)) * (uint32_t)sizeof(T);
-  }
-  __device__ __forceinline__ uint32_t rowo(int x, int y, int z) const {
-    return (ox<T>(x & ~((1 << Blk<T>::LX) - 1)) + oy<T>(y, nbx) + oz<T>(z, nbxy)) * (uint32_t)sizeof(T);
-  }
-  __device__ __forceinline__ const uint8_t* base() const { return reinterpret_cast<const uint8_t*>(d); }
-
-  __device__ __forceinline__ float value(const T* __restrict__ dd, int nx, int ny, int nz, bool e, V3 pos) {
-    d = dd; n[0] = nx; n[1] = ny; n[2] = nz; edge = e; p = pos;
+  __device__ __forceinline__ float value(const T* __restrict__ dd, int nx, int ny, int nz, bool, V3 p) {
+    base = reinterpret_cast<const uint8_t*>(dd);
     const float pc[3] = {p.x, p.y, p.z};
+    const int n[3] = {nx, ny, nz};
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const float s = fminf(fmaxf(pc[a], 0.0f), 1.0f), u = s * (float)n[a] - 0.5f, fl = floorf(u);
@@ -382,7 +374,10 @@ struct CrossSampler<T, true> {
     }
     nbx = nblocks((uint32_t)nx, Blk<T>::LX);
     nbxy = nbx * nblocks((uint32_t)ny, 2);
+    const RowSteps R(nbx, nbxy);
+    row0 = R.at(ic[1], ic[2]);
     const int xs = ic[0] - 1, sx = xs & ((1 << Blk<T>::LX) - 1);
+    const uint32_t r00 = row0 + ((uint32_t)(xs >> Blk<T>::LX) << 8), dy = R.yp1(ic[1]), dz = R.zp1(ic[2]);
     // the four loads are issued before the first of them is used: near 128 VGPRs
     // the scheduler otherwise waits for each in turn to save registers (64.0
     // against 54.2 ms for 16 lit 2D 1080p frames of 1024^3)
@@ -390,7 +385,7 @@ struct CrossSampler<T, true> {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int k = 0; k < 2; ++k) w[j][k] = run4_load<T>(base(), rowo(xs, ic[1] + j, ic[2] + k), sx);
+      for (int k = 0; k < 2; ++k) w[j][k] = run4_load<T>(base, r00 + (j ? dy : 0u) + (k ? dz : 0u), sx);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -410,20 +405,24 @@ struct CrossSampler<T, true> {
   // every tap of an interior sample is unclamped (1 <= floor(u) and
   // floor(u) + 2 < n on every axis put p +- 1/n inside [0, 1]): the index form
   __device__ __forceinline__ V3 gradient(V3) const {
+    const RowSteps R(nbx, nbxy);
+    const uint32_t v00 = row0 + ox<T>(ic[0]) * (uint32_t)sizeof(T);   // voxel (x0, y0, z0)
+    const uint32_t dy = R.yp1(ic[1]), dz = R.zp1(ic[2]);
+    const uint32_t ym = v00 + R.ym1(ic[1]), yp = v00 + R.yp2(ic[1]), zm = v00 + R.zm1(ic[2]), zp = v00 + R.zp2(ic[2]);
     float yl[2][2], yr[2][2], zl[2][2], zr[2][2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       uint32_t a[2], b[2];
-      run2<T>(base(), vox(ic[0], ic[1] - 1, ic[2] + k), a);
-      run2<T>(base(), vox(ic[0], ic[1] + 2, ic[2] + k), b);
+      run2<T>(base, ym + (k ? dz : 0u), a);
+      run2<T>(base, yp + (k ? dz : 0u), b);
       yl[0][k] = (float)a[0]; yl[1][k] = (float)a[1];
       yr[0][k] = (float)b[0]; yr[1][k] = (float)b[1];
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       uint32_t a[2], b[2];
-      run2<T>(base(), vox(ic[0], ic[1] + j, ic[2] - 1), a);
-      run2<T>(base(), vox(ic[0], ic[1] + j, ic[2] + 2), b);
+      run2<T>(base, zm + (j ? dy : 0u), a);
+      run2<T>(base, zp + (j ? dy : 0u), b);
       zl[0][j] = (float)a[0]; zl[1][j] = (float)a[1];
       zr[0][j] = (float)b[0]; zr[1][j] = (float)b[1];
     }
