@@ -106,3 +106,41 @@ def test_brick_uploaded_again_reaches_every_context():
         batch.Render()
         assert np.array_equal(batch.Frame(0), fb)
         batch.close()
+
+
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16])
+@pytest.mark.parametrize("again", [1, 3, 27])
+def test_cell_grid_after_uploads(dtype, again):
+    """Bricks uploaded again after the grid was made (one, a few, most): the grid
+    equals that of the same bricks handed over at first, and the frame too."""
+    dims, core = (40, 44, 36), 14
+    grid = [-(-d // core) for d in dims]
+    rng = np.random.default_rng(11)
+    keys, first, second = [], [], []
+    for z in range(grid[2]):
+        for y in range(grid[1]):
+            for x in range(grid[0]):
+                n = [(core if p + 1 < g or d % core == 0 else d % core) + 2 for p, g, d in zip((x, y, z), grid, dims)]
+                keys.append((0, len(keys), (0.0, float(np.iinfo(dtype).max))))
+                first.append(rng.integers(0, 3, n[::-1]).astype(dtype))
+                second.append(rng.integers(0, np.iinfo(dtype).max, n[::-1]).astype(dtype))
+    pick = rng.permutation(len(keys))[:min(again, len(keys))]
+    out = []
+    for late in (True, False):
+        with HIPRaycaster(0) as r:
+            r.SetBricks(dtype, dims, (core + 2,) * 3, 1, keys, lod_count=1)
+            for i, b in enumerate(first):
+                r.UploadBrick(0, i, b if late or i not in pick else second[i])
+            r.Set1DTrans(table("ramp"))
+            r.SetRendermode(RM_1DTRANS)
+            r.SetUseLighting(False)
+            r.SetViewParameters(45.0, 0.01, 1000.0)
+            r.SetViewPosition((0.0, 0.0, 1.8))
+            r.Resize(80, 60)
+            if late:
+                r.Paint()
+                for i in pick:
+                    r.UploadBrick(0, int(i), second[i])
+            out.append((r.Paint(), r.CellGrid()))
+    assert np.array_equal(out[0][1], out[1][1])
+    assert np.array_equal(out[0][0], out[1][0])

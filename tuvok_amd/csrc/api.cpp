@@ -1179,6 +1179,52 @@ int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads) {
   if (e != hipSuccess) return hipfail(c, "cell grid", e);
   G.d = (uint32_t*)G.hold.get();
   G.base = std::move(base);
+  G.stale.clear();
+  G.ready.store(true, std::memory_order_release);
+  return TVK_OK;
+}
+
+int remake_cells(tvk_ctx* c, CellGrid& G) {
+  const Layout& L = c->L;
+  std::sort(G.stale.begin(), G.stale.end());
+  G.stale.erase(std::unique(G.stale.begin(), G.stale.end()), G.stale.end());
+  const size_t n = G.stale.size();
+  if (8 * n >= L.toc.size()) return make_cells(c, G, nullptr);
+  // one brick at a time through a quad buffer of the largest
+  const uint32_t per = L.bpv == 1 ? 256u : 128u, h = L.bpv == 1 ? 2u : 1u;   // elements and quads of a block
+  std::vector<GatherBrick> gb(n);
+  std::vector<uint32_t> base(n);
+  uint64_t most = 0;
+  for (size_t i = 0; i < n; ++i) {
+    const TocBrick& t = L.toc[G.stale[i]];
+    for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)t.coords[k]; gb[i].n[k] = t.size[k]; }
+    gb[i].offset = t.offset;
+    base[i] = G.base[G.stale[i]];
+    most = std::max<uint64_t>(most, t.count);
+  }
+  std::shared_ptr<void> gb_hold, base_hold, quad_hold;
+  hipError_t e = device_block(&gb_hold, n * sizeof(GatherBrick));
+  if (e == hipSuccess) e = device_block(&base_hold, n * sizeof(uint32_t));
+  if (e == hipSuccess) e = device_block(&quad_hold, (size_t)(most / per) * h * sizeof(uint32_t));
+  if (e != hipSuccess) return hipfail(c, "cell grid", e);
+  const GatherBrick* const d_gb = (const GatherBrick*)gb_hold.get();
+  e = hipMemcpyAsync(gb_hold.get(), gb.data(), n * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(base_hold.get(), base.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
+  for (size_t i = 0; i < n && e == hipSuccess; ++i) {
+    // the kernels index quads by the brick's place in the pool: the buffer
+    // stands where that brick's quads would be
+    const uintptr_t shift = (uintptr_t)(gb[i].offset / per) * h * sizeof(uint32_t);
+    uint32_t* const quads = (uint32_t*)((uintptr_t)quad_hold.get() - shift);
+    const uint32_t cells = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
+    e = launch_minmax(c->d_pool, L.bpv, d_gb + i, 1, (uint32_t)L.toc[G.stale[i]].count, nullptr, quads, c->stream);
+    if (e == hipSuccess)
+      e = launch_cells(quads, L.bpv, d_gb + i, (const uint32_t*)base_hold.get() + i, 1, cells, G.d, c->stream);
+  }
+  const hipError_t se = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = se;
+  if (e != hipSuccess) return hipfail(c, "cell grid", e);
+  G.stale.clear();
   G.ready.store(true, std::memory_order_release);
   return TVK_OK;
 }
@@ -1190,7 +1236,8 @@ int ensure_cells(tvk_ctx* c) {
   CellGrid& G = *c->cells;
   if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
   std::lock_guard<std::mutex> lk(G.mu);
-  return G.ready.load(std::memory_order_acquire) ? TVK_OK : make_cells(c, G, nullptr);
+  if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
+  return G.d && !G.stale.empty() ? remake_cells(c, G) : make_cells(c, G, nullptr);
 }
 
 void brick_tf_stats(tvk_ctx* c, FrameBrick& fb) {

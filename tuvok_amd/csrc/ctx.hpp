@@ -96,10 +96,12 @@ struct PoolState {
 // from which the march knows the stretches of a ray that cannot contribute.  Made
 // with the bricks, or on first use for bricks handed over one by one; shared by
 // the contexts that share the dataset.  A brick uploaded again clears `ready` for
-// all of them; the next use makes the words again in place.
+// all of them; the next use makes that brick's words again in place (an eighth
+// of the bricks or more: all of them).
 struct CellGrid {
-  std::mutex mu;                // held while it is made
+  std::mutex mu;                // held while it is made, and for stale
   std::atomic<bool> ready{false};
+  std::vector<uint32_t> stale;  // TOC bricks uploaded again since it was made
   std::shared_ptr<void> hold;
   uint32_t* d = nullptr;
   std::vector<uint32_t> base;   // first cell of each TOC brick
@@ -309,6 +311,8 @@ int ensure_cells(tvk_ctx* c);
 // The cell grid from quad ranges of every brick (quads, or null: read from the
 // pool), stream-ordered; needs G.mu.
 int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads);
+// The words of the stale bricks alone; needs G.mu and a grid made before.
+int remake_cells(tvk_ctx* c, CellGrid& G);
 inline size_t quad_words(const Layout& L) { return (size_t)(L.pool_elems / (L.bpv == 1 ? 256u : 128u)) * (L.bpv == 1 ? 2u : 1u); }
 // the cell grid as the kernels read it; null while it is not made, for
 // compatibility textures and for a budgeted pool
