@@ -688,8 +688,9 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
       // clamped taps) is never skipped.  Skipped samples only advance pos (and
       // cur) by the march's own additions, so everything after them is the same
       // bit for bit: a transparent sample adds 0 to the colour and alpha, one
-      // below the isovalue moves on.  On the 1024^3 phantom (84% transparent
-      // samples) a probe goes by 15 of them.
+      // below the isovalue moves on.  Four lit 1D 1080p frames of the 1024^3
+      // phantom (84% transparent samples): 8.6 -> 4.4 ms; a 2048^3 isosurface
+      // 2.9 -> 1.15 ms.
       constexpr bool SKIP = LEARN == 0 && MODE != 1;
       const uint32_t* __restrict__ cg = nullptr;
       int sncx = 0, sncy = 0;
