@@ -257,7 +257,11 @@ typedef struct {
 } tvk_uvf_info;
 int tvk_open_uvf(tvk_ctx* ctx, const char* path, uint64_t budget_bytes, tvk_uvf_info* info);
 /* One brick's payload, Dataset::GetBrick (IO/Dataset.h:93-100): the reference
- * layout, x fastest, stored size incl. overlap (bytes must match). */
+ * layout, x fastest, stored size incl. overlap (bytes must match).  A brick may be
+ * uploaded again: the contexts that share the dataset see it from their next frame
+ * on.  Contexts may be used on threads of their own; a frame that is rendered or
+ * queued while a brick of its dataset is uploaded may show either content of that
+ * brick, voxel by voxel. */
 int tvk_upload_brick(tvk_ctx* ctx, uint32_t lod, uint64_t index, const void* data, size_t bytes);
 /* Holds the current dataset within budget_bytes of HBM (as above; its bricks are
  * copied to pinned host memory first), or, with 0, makes every brick resident

@@ -1,6 +1,8 @@
 """The march that goes by stretches that cannot contribute (datasets with a cell
 grid) against the march that samples every step: a budgeted pool has no grid, so
 its frames, sample counts and hits must equal the resident pool's bit for bit."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -144,3 +146,66 @@ def test_cell_grid_after_uploads(dtype, again):
             out.append((r.Paint(), r.CellGrid()))
     assert np.array_equal(out[0][1], out[1][1])
     assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("learned", [False, True])
+def test_uploads_beside_another_contexts_frames(learned):
+    """One thread uploads the bricks of a shared dataset again (the same voxels) and
+    renders, so that the grid is made anew each time; frames and batches of another
+    context on another thread stay what they were."""
+    core = 14
+    vol = sparse_volume((2 * core, core, core), np.uint8, 3)
+    with HIPRaycaster(0) as ref:
+        ref.LoadVolume(vol, (core + 2,) * 3, 1, max_lods=1)
+        bricks = [ref.GetBrick(i) for i in range(2)]
+    with HIPRaycaster(0) as a, HIPRaycaster(0) as b:
+        a.SetBricks(np.uint8, (2 * core, core, core), (core + 2,) * 3, 1, [(0, i, (0.0, 255.0)) for i in range(2)],
+                    lod_count=1)
+        for i in range(2):
+            a.UploadBrick(0, i, bricks[i])
+        b.ShareDataset(a)
+        for x in (a, b):
+            x.Set1DTrans(table("ramp"))
+            x.SetRendermode(RM_1DTRANS)
+            x.SetUseLighting(False)
+            x.SetViewParameters(45.0, 0.01, 1000.0)
+            x.SetViewPosition((0.0, 0.0, 1.8))
+            x.Resize(64, 48)
+        if learned:
+            b.SetStepProposal(None, fixed_log2=0)
+        want = b.Paint()
+        assert want[..., 3].max() > 0
+        batch = RenderBatch(0)
+        batch.Add(b, None, 64, 48)
+        batch.Render()
+        want_batch = batch.Frame(0)
+        bad, rounds = [], [0, 0]
+
+        def upload():
+            try:
+                for k in range(60):
+                    a.UploadBrick(0, k % 2, bricks[k % 2])
+                    a.Paint()
+                    rounds[0] += 1
+            except Exception as e:
+                bad.append(e)
+
+        def render():
+            try:
+                for k in range(60):
+                    if not np.array_equal(b.Paint(), want):
+                        bad.append(k)
+                    batch.Render()
+                    if not np.array_equal(batch.Frame(0), want_batch):
+                        bad.append(("batch", k))
+                    rounds[1] += 1
+            except Exception as e:
+                bad.append(e)
+
+        ts = [threading.Thread(target=f) for f in (upload, render)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        batch.close()
+        assert not bad and rounds == [60, 60]

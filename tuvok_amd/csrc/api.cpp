@@ -1143,14 +1143,15 @@ int learn_prepare(tvk_ctx* c) {
 int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads) {
   const Layout& L = c->L;
   std::vector<GatherBrick> gb(L.toc.size());
-  std::vector<uint32_t> base(L.toc.size(), 0);
+  uint32_t* words = G.words.load(std::memory_order_relaxed);
+  if (!words) G.base.assign(L.toc.size(), 0);   // no other thread reads it yet
   uint64_t total = 0;
   uint32_t max_cells = 0, max_vox = 0;
   for (size_t i = 0; i < L.toc.size(); ++i) {
     for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)L.toc[i].coords[k]; gb[i].n[k] = L.toc[i].size[k]; }
     gb[i].offset = L.toc[i].offset;
     const uint32_t nc = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
-    base[i] = (uint32_t)total;
+    if (!words) G.base[i] = (uint32_t)total;
     total += nc;
     max_cells = std::max(max_cells, nc);
     max_vox = std::max(max_vox, (uint32_t)L.toc[i].count);
@@ -1159,26 +1160,26 @@ int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads) {
   std::shared_ptr<void> gb_hold, base_hold, quad_hold;
   hipError_t e = hipSuccess;
   if (!G.hold) e = device_block(&G.hold, std::max<uint64_t>(total, 1) * sizeof(uint32_t));
+  words = (uint32_t*)G.hold.get();
   if (e == hipSuccess) e = device_block(&gb_hold, gb.size() * sizeof(GatherBrick));
-  if (e == hipSuccess) e = device_block(&base_hold, base.size() * sizeof(uint32_t));
+  if (e == hipSuccess) e = device_block(&base_hold, G.base.size() * sizeof(uint32_t));
   if (e == hipSuccess && !quads) e = device_block(&quad_hold, quad_words(L) * sizeof(uint32_t));
   if (e != hipSuccess) return hipfail(c, "cell grid", e);
   GatherBrick* const d_gb = (GatherBrick*)gb_hold.get();
   e = hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(base_hold.get(), base.data(), base.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
+    e = hipMemcpyAsync(base_hold.get(), G.base.data(), G.base.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess && !quads) {
     e = launch_minmax(c->d_pool, L.bpv, d_gb, (uint32_t)gb.size(), max_vox, nullptr, (uint32_t*)quad_hold.get(), c->stream);
     quads = (const uint32_t*)quad_hold.get();
   }
   if (e == hipSuccess)
     e = launch_cells(quads, L.bpv, d_gb, (const uint32_t*)base_hold.get(), (uint32_t)gb.size(), max_cells,
-                     (uint32_t*)G.hold.get(), c->stream);
+                     words, c->stream);
   const hipError_t se = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) e = se;
   if (e != hipSuccess) return hipfail(c, "cell grid", e);
-  G.d = (uint32_t*)G.hold.get();
-  G.base = std::move(base);
+  G.words.store(words, std::memory_order_release);
   G.stale.clear();
   G.ready.store(true, std::memory_order_release);
   return TVK_OK;
@@ -1219,7 +1220,8 @@ int remake_cells(tvk_ctx* c, CellGrid& G) {
     const uint32_t cells = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
     e = launch_minmax(c->d_pool, L.bpv, d_gb + i, 1, (uint32_t)L.toc[G.stale[i]].count, nullptr, quads, c->stream);
     if (e == hipSuccess)
-      e = launch_cells(quads, L.bpv, d_gb + i, (const uint32_t*)base_hold.get() + i, 1, cells, G.d, c->stream);
+      e = launch_cells(quads, L.bpv, d_gb + i, (const uint32_t*)base_hold.get() + i, 1, cells,
+                       G.words.load(std::memory_order_relaxed), c->stream);
   }
   const hipError_t se = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) e = se;
@@ -1237,7 +1239,7 @@ int ensure_cells(tvk_ctx* c) {
   if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
   std::lock_guard<std::mutex> lk(G.mu);
   if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
-  return G.d && !G.stale.empty() ? remake_cells(c, G) : make_cells(c, G, nullptr);
+  return G.words.load(std::memory_order_relaxed) && !G.stale.empty() ? remake_cells(c, G) : make_cells(c, G, nullptr);
 }
 
 void brick_tf_stats(tvk_ctx* c, FrameBrick& fb) {
@@ -1290,7 +1292,6 @@ void fill_shade(const tvk_ctx* c, ShadeConst& S) {
   S.tfst = c->d_tfst;
   S.tfst_n = c->tfst.n;
   S.tfst_levels = c->tfst.levels;
-  S.cells = cells_device(c);
   S.overlap = (int)c->L.overlap;
 }
 
@@ -1382,7 +1383,7 @@ int render_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_
     int rc = learn_prepare(c);
     if (rc) return rc;
   }
-  const uint32_t* const cells = fixed ? cells_device(c) : cells_for_render(c);
+  const uint32_t* const cells = learn > 0 ? cells_for_learn(c) : (fixed ? cells_device(c) : cells_for_render(c));
   c->h_list.clear();
   c->h_views.assign((size_t)nviews, ViewConst{});
   std::vector<PlannedBrick> planned;
@@ -1665,7 +1666,8 @@ int tvk_cell_grid(tvk_ctx* c, uint32_t* out, uint64_t cap, uint64_t* n) {
   }
   *n = total;
   if (out && cap) {
-    HIPCHK(c, hipMemcpy(out, G.d, std::min(cap, total) * sizeof(uint32_t), hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpy(out, G.words.load(std::memory_order_acquire), std::min(cap, total) * sizeof(uint32_t),
+                        hipMemcpyDeviceToHost));
   }
   return TVK_OK;
 }

@@ -167,13 +167,14 @@ int plan_batch(tvk_batch* b, uint32_t* bricks_total) {
       if (!rc) {
         plan_frame(c->L, c->minmax, c->range_max, V, pp, planned);
         make_frame_bricks(c->L, V, pp, planned, P[i].list, compat_dims(c), compat_offsets(c));
-        P[i].cells = cells_for_render(c);
-        brick_cells(c, P[i].cells, P[i].list.data(), P[i].list.size());
-        if (b->net && c->P.mode != TVK_RM_ISOSURFACE) {
-          rc = learn_prepare(c);
-          if (!rc)
-            for (FrameBrick& fb : P[i].list) brick_tf_stats(c, fb);
+        const bool learn = b->net && c->P.mode != TVK_RM_ISOSURFACE;
+        if (learn) rc = learn_prepare(c);
+        if (!rc) {
+          P[i].cells = learn ? cells_for_learn(c) : cells_for_render(c);
+          brick_cells(c, P[i].cells, P[i].list.data(), P[i].list.size());
         }
+        if (!rc && learn)
+          for (FrameBrick& fb : P[i].list) brick_tf_stats(c, fb);
       }
     }
     if (rc) return bfail(b, rc, "request " + std::to_string(i) + ": " + c->err);

@@ -95,16 +95,18 @@ struct PoolState {
 // Cell grid of a dataset: per brick, the (min, max) of its cells (tvk_types.hpp),
 // from which the march knows the stretches of a ray that cannot contribute.  Made
 // with the bricks, or on first use for bricks handed over one by one; shared by
-// the contexts that share the dataset.  A brick uploaded again clears `ready` for
+// the contexts that share the dataset, whatever thread each is used on.  What a
+// render holds on to never moves: `words` is set once and `base`, which the layout
+// alone decides, is filled before that.  A brick uploaded again clears `ready` for
 // all of them; the next use makes that brick's words again in place (an eighth
 // of the bricks or more: all of them).
 struct CellGrid {
-  std::mutex mu;                // held while it is made, and for stale
-  std::atomic<bool> ready{false};
-  std::vector<uint32_t> stale;  // TOC bricks uploaded again since it was made
+  std::mutex mu;                // held while the words are made, and for stale
+  std::atomic<bool> ready{false};   // the words are those of the bricks as they are
+  std::atomic<uint32_t*> words{nullptr};
+  std::vector<uint32_t> base;   // first cell of each TOC brick (read where words is set)
+  std::vector<uint32_t> stale;  // TOC bricks uploaded again since the words were made
   std::shared_ptr<void> hold;
-  uint32_t* d = nullptr;
-  std::vector<uint32_t> base;   // first cell of each TOC brick
 };
 }  // namespace tvk
 
@@ -126,7 +128,7 @@ struct tvk_ctx {
   void* d_pool = nullptr;
   std::shared_ptr<void> pool_hold;   // owns d_pool; shared by contexts that share the dataset
   std::shared_ptr<void> lin_hold;    // owns d_lin
-  std::shared_ptr<tvk::CellGrid> cells;   // created with the pool, filled on first learned use
+  std::shared_ptr<tvk::CellGrid> cells;   // created with the pool
   std::shared_ptr<tvk::PoolState> pst;    // null: every brick resident at its TOC offset
   // bricks declared by tvk_set_bricks (resident pool) whose payload has not
   // arrived yet: rendering waits for all of them
@@ -317,7 +319,9 @@ inline size_t quad_words(const Layout& L) { return (size_t)(L.pool_elems / (L.bp
 // the cell grid as the kernels read it; null while it is not made, for
 // compatibility textures and for a budgeted pool
 inline const uint32_t* cells_device(const tvk_ctx* c) {
-  return !compat_active(c) && !c->pst && c->cells && c->cells->ready.load(std::memory_order_acquire) ? c->cells->d : nullptr;
+  return !compat_active(c) && !c->pst && c->cells && c->cells->ready.load(std::memory_order_acquire)
+             ? c->cells->words.load(std::memory_order_acquire)
+             : nullptr;
 }
 // the step network as the kernels read it (false when s is null)
 bool stepnet_device(const struct tvk_stepnet* s, StepNetDev* out);
@@ -337,7 +341,7 @@ int pool_set_budget(tvk_ctx* c, uint64_t budget_bytes);
 // Copies bricks [first, first+n) in the reference layout to host memory.
 int pool_download(tvk_ctx* c, size_t first, size_t n, void* host, size_t bytes);
 inline bool budgeted(const tvk_ctx* c) { return c->pst != nullptr; }
-// first cells of the listed bricks (cells: cells_device's, may be null)
+// first cells of the listed bricks (cells: the grid's words, or null)
 inline void brick_cells(const tvk_ctx* c, const uint32_t* cells, FrameBrick* fb, size_t n) {
   for (size_t i = 0; i < n; ++i) fb[i].cells = cells ? c->cells->base[fb[i].toc] : 0u;
 }
@@ -350,6 +354,9 @@ inline const uint32_t* cells_for_render(tvk_ctx* c) {
   }
   return cells_device(c);
 }
+// The grid that a learned march reads, after learn_prepare has made it: also where
+// another context's upload has cleared `ready` since, a brick's former words then.
+inline const uint32_t* cells_for_learn(const tvk_ctx* c) { return c->cells->words.load(std::memory_order_acquire); }
 // a frame of a budgeted dataset (fixed step, any mode)
 int render_budget_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_stats* st);
 
