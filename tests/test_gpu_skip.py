@@ -1,12 +1,13 @@
 """The march that goes by stretches that cannot contribute (datasets with a cell
 grid) against the march that samples every step: a budgeted pool has no grid, so
 its frames, sample counts and hits must equal the resident pool's bit for bit."""
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
 
-from tuvok_amd import RM_1DTRANS, RM_ISOSURFACE, HIPRaycaster, RenderBatch, rotation_y
+from tuvok_amd import RM_1DTRANS, RM_2DTRANS, RM_ISOSURFACE, HIPRaycaster, RenderBatch, _abi, rotation_y
 
 pytestmark = pytest.mark.gpu
 
@@ -209,3 +210,35 @@ def test_uploads_beside_another_contexts_frames(learned):
             t.join()
         batch.close()
         assert not bad and rounds == [60, 60]
+
+
+def test_2d_frames_make_no_grid():
+    """A fixed-step 2D frame of bricks handed over one by one neither reads nor makes
+    the cell grid (its ranges of 4^3 voxels are 8 MiB here); a 1D frame makes it."""
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert _abi.load().hipMemGetInfo(C.byref(a), C.byref(b)) == 0   # of the library's own HIP runtime
+        return a.value
+
+    core, g = 126, 4
+    tf2 = np.full((16, 16, 4), 3, np.uint8)
+    with HIPRaycaster(0) as r:
+        r.LoadVolume(np.full((20, 20, 20), 9, np.uint8), (18,) * 3, 1, max_lods=1)
+        r.Set2DTrans(tf2)
+        r.Set1DTrans(table("ramp"))
+        r.SetRendermode(RM_2DTRANS)
+        r.SetUseLighting(False)
+        r.SetViewParameters(45.0, 0.01, 1000.0)
+        r.SetViewPosition((0.0, 0.0, 1.8))
+        r.Resize(64, 64)
+        r.Paint()   # the frame's own buffers
+        r.SetBricks(np.uint8, (core * g,) * 3, (core + 2,) * 3, 1, [(0, i, (0.0, 255.0)) for i in range(g ** 3)],
+                    lod_count=1)
+        brick = np.full((core + 2,) * 3, 7, np.uint8)
+        for i in range(g ** 3):
+            r.UploadBrick(0, i, brick)
+        before = free()
+        assert r.Paint()[..., 3].max() > 0
+        r.UploadBrick(0, 5, brick)
+        r.Paint()
+        assert before - free() <= 4 << 20

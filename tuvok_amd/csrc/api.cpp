@@ -1180,16 +1180,17 @@ int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads) {
   if (e == hipSuccess) e = se;
   if (e != hipSuccess) return hipfail(c, "cell grid", e);
   G.words.store(words, std::memory_order_release);
-  G.stale.clear();
+  G.stale.assign(L.toc.size(), 0);
   G.ready.store(true, std::memory_order_release);
   return TVK_OK;
 }
 
 int remake_cells(tvk_ctx* c, CellGrid& G) {
   const Layout& L = c->L;
-  std::sort(G.stale.begin(), G.stale.end());
-  G.stale.erase(std::unique(G.stale.begin(), G.stale.end()), G.stale.end());
-  const size_t n = G.stale.size();
+  std::vector<uint32_t> list;
+  for (uint32_t t = 0; t < L.toc.size(); ++t)
+    if (G.stale[t]) list.push_back(t);
+  const size_t n = list.size();
   if (8 * n >= L.toc.size()) return make_cells(c, G, nullptr);
   // one brick at a time through a quad buffer of the largest
   const uint32_t per = L.bpv == 1 ? 256u : 128u, h = L.bpv == 1 ? 2u : 1u;   // elements and quads of a block
@@ -1197,10 +1198,10 @@ int remake_cells(tvk_ctx* c, CellGrid& G) {
   std::vector<uint32_t> base(n);
   uint64_t most = 0;
   for (size_t i = 0; i < n; ++i) {
-    const TocBrick& t = L.toc[G.stale[i]];
+    const TocBrick& t = L.toc[list[i]];
     for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)t.coords[k]; gb[i].n[k] = t.size[k]; }
     gb[i].offset = t.offset;
-    base[i] = G.base[G.stale[i]];
+    base[i] = G.base[list[i]];
     most = std::max<uint64_t>(most, t.count);
   }
   std::shared_ptr<void> gb_hold, base_hold, quad_hold;
@@ -1218,7 +1219,7 @@ int remake_cells(tvk_ctx* c, CellGrid& G) {
     const uintptr_t shift = (uintptr_t)(gb[i].offset / per) * h * sizeof(uint32_t);
     uint32_t* const quads = (uint32_t*)((uintptr_t)quad_hold.get() - shift);
     const uint32_t cells = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
-    e = launch_minmax(c->d_pool, L.bpv, d_gb + i, 1, (uint32_t)L.toc[G.stale[i]].count, nullptr, quads, c->stream);
+    e = launch_minmax(c->d_pool, L.bpv, d_gb + i, 1, (uint32_t)L.toc[list[i]].count, nullptr, quads, c->stream);
     if (e == hipSuccess)
       e = launch_cells(quads, L.bpv, d_gb + i, (const uint32_t*)base_hold.get() + i, 1, cells,
                        G.words.load(std::memory_order_relaxed), c->stream);
@@ -1226,7 +1227,7 @@ int remake_cells(tvk_ctx* c, CellGrid& G) {
   const hipError_t se = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) e = se;
   if (e != hipSuccess) return hipfail(c, "cell grid", e);
-  G.stale.clear();
+  G.stale.assign(L.toc.size(), 0);
   G.ready.store(true, std::memory_order_release);
   return TVK_OK;
 }
@@ -1239,7 +1240,7 @@ int ensure_cells(tvk_ctx* c) {
   if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
   std::lock_guard<std::mutex> lk(G.mu);
   if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
-  return G.words.load(std::memory_order_relaxed) && !G.stale.empty() ? remake_cells(c, G) : make_cells(c, G, nullptr);
+  return G.words.load(std::memory_order_relaxed) ? remake_cells(c, G) : make_cells(c, G, nullptr);
 }
 
 void brick_tf_stats(tvk_ctx* c, FrameBrick& fb) {
@@ -1383,7 +1384,10 @@ int render_impl(tvk_ctx* c, int nviews, const float* rots, float* host_out, tvk_
     int rc = learn_prepare(c);
     if (rc) return rc;
   }
-  const uint32_t* const cells = learn > 0 ? cells_for_learn(c) : (fixed ? cells_device(c) : cells_for_render(c));
+  const uint32_t* const cells = learn > 0                  ? cells_for_learn(c)
+                                : fixed && march_skips(c) ? cells_device(c)
+                                : fixed                    ? nullptr
+                                                           : cells_for_render(c);
   c->h_list.clear();
   c->h_views.assign((size_t)nviews, ViewConst{});
   std::vector<PlannedBrick> planned;

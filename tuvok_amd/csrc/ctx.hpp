@@ -105,7 +105,7 @@ struct CellGrid {
   std::atomic<bool> ready{false};   // the words are those of the bricks as they are
   std::atomic<uint32_t*> words{nullptr};
   std::vector<uint32_t> base;   // first cell of each TOC brick (read where words is set)
-  std::vector<uint32_t> stale;  // TOC bricks uploaded again since the words were made
+  std::vector<uint8_t> stale;   // per TOC brick: uploaded again since the words were made
   std::shared_ptr<void> hold;
 };
 }  // namespace tvk
@@ -345,9 +345,14 @@ inline bool budgeted(const tvk_ctx* c) { return c->pst != nullptr; }
 inline void brick_cells(const tvk_ctx* c, const uint32_t* cells, FrameBrick* fb, size_t n) {
   for (size_t i = 0; i < n; ++i) fb[i].cells = cells ? c->cells->base[fb[i].toc] : 0u;
 }
-// The cell grid for a render of the context, made if that has not happened; null
-// where the bricks have none (a march without it samples every step).
+// Whether a fixed-step frame of the context reads the cell grid: the 1D and
+// isosurface marches do, the 2D one samples every step.
+inline bool march_skips(const tvk_ctx* c) { return c->P.mode != TVK_RM_2DTRANS; }
+// The cell grid for a fixed-step render of the context, made if that has not
+// happened; null where the march does not read it or the bricks have none (a march
+// without it samples every step).
 inline const uint32_t* cells_for_render(tvk_ctx* c) {
+  if (!march_skips(c)) return nullptr;
   if (!budgeted(c) && !compat_active(c) && c->cells && !c->cells->ready.load(std::memory_order_acquire)) {
     const std::string msg = c->err;
     if (ensure_cells(c) != TVK_OK) { (void)hipGetLastError(); c->err = msg; }

@@ -631,7 +631,7 @@ int tvk_upload_brick(tvk_ctx* c, uint32_t lod, uint64_t index, const void* data,
   c->cp = tvk_ctx::CompatPool{};   // made again from the new contents on the next render
   if (c->cells) {   // the brick's cells are made again on next use
     std::lock_guard<std::mutex> lk(c->cells->mu);
-    if (c->cells->words.load(std::memory_order_relaxed)) c->cells->stale.push_back(t);
+    if (c->cells->words.load(std::memory_order_relaxed)) c->cells->stale[t] = 1;
     c->cells->ready.store(false, std::memory_order_release);
   }
   return TVK_OK;
