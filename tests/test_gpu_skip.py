@@ -32,7 +32,8 @@ def table(kind):
     t = np.zeros((256, 4), np.uint8)
     t[:, :3] = np.arange(256)[:, None]
     t[:, 3] = {"ramp": np.maximum(np.arange(256) - 60, 0) // 2, "gaps": np.where(np.arange(256) % 64 > 50, 30, 0),
-               "all": 20, "last": np.where(np.arange(256) == 255, 200, 0)}[kind]
+               "all": 20, "last": np.where(np.arange(256) == 255, 200, 0), "none": 0,
+               "low": np.where(np.arange(256) < 3, 2, 0)}[kind]
     return t
 
 
@@ -63,6 +64,7 @@ def test_skipped_stretches(dims, brick, ov, edge, dtype):
         for mode, tf, lit, srm, ert in ((RM_1DTRANS, "ramp", False, 1.0, 0.0), (RM_1DTRANS, "ramp", True, 2.0, 2.0 ** -11),
                                         (RM_1DTRANS, "gaps", True, 1.0, 0.0), (RM_1DTRANS, "gaps", False, 0.7, 2.0 ** -11),
                                         (RM_1DTRANS, "all", False, 1.0, 0.0), (RM_1DTRANS, "last", True, 1.0, 0.0),
+                                        (RM_1DTRANS, "low", False, 1.0, 0.0), (RM_1DTRANS, "none", True, 1.0, 0.0),
                                         (RM_ISOSURFACE, None, True, 1.0, 0.0), (RM_ISOSURFACE, None, True, 3.0, 2.0 ** -11)):
             for x in (r, q):
                 if tf:
@@ -76,7 +78,7 @@ def test_skipped_stretches(dims, brick, ov, edge, dtype):
             assert np.array_equal(a, b), (mode, tf, lit, srm)
             if mode == RM_1DTRANS or ert == 0.0:   # the hit skip of a frame rendered in parts sees only its part
                 assert na == nb
-            assert tf == "last" or a[..., 3].max() > 0   # only the very top value: samples may miss it
+            assert tf in ("last", "none") or a[..., 3].max() > 0   # only the very top value: samples may miss it
 
 
 def test_brick_uploaded_again_reaches_every_context():

@@ -821,6 +821,9 @@ int tvk_set_tf1d(tvk_ctx* c, const uint8_t* rgba8, int n) {
   std::vector<uint16_t> next((size_t)n);
   for (int i = n - 1; i >= 0; --i)
     next[(size_t)i] = rgba8[4 * (size_t)i + 3] ? (uint16_t)i : (i + 1 < n ? next[(size_t)i + 1] : (uint16_t)0xffff);
+  c->tf1d_first = std::min((int)next[0], n);
+  c->tf1d_clear = false;
+  for (int i = 0; i < n; ++i) c->tf1d_clear = c->tf1d_clear || rgba8[4 * (size_t)i + 3] == 0;
   // texture1D of the RGBA8 table returns byte/255 (GL_NEAREST): expand once
   const std::vector<float4> f = unorm_table(rgba8, (size_t)n);
   HIPCHK(c, hipMemcpyAsync(c->d_tf1d, c->tf1d.data(), 4 * (size_t)n, hipMemcpyHostToDevice, c->stream));
@@ -1274,6 +1277,7 @@ void fill_shade(const tvk_ctx* c, ShadeConst& S) {
   S.tf2_cols = c->d_tf2cols;
   S.tf1_next = c->d_tf1next;
   S.tf_n = c->tf1d_n;
+  S.tf1_first = c->tf1d_first;
   S.tf_w = c->tf2d_w;
   S.tf_h = c->tf2d_h;
   S.tf_scale = tf_scale_of(c);

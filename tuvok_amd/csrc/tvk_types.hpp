@@ -85,6 +85,7 @@ struct ShadeConst {
   const float4* tf2f;           // 2D TF as float4 (byte / 255), tf_w x tf_h
   const uint64_t* tf2_cols;     // bit x: value column x of the 2D TF has a non-zero alpha (64 words)
   const uint16_t* tf1_next;     // per 1D TF entry: the first entry from it on with a non-zero alpha (0xffff: none)
+  int tf1_first;                // first 1D TF entry with a non-zero alpha (tf_n: none)
   int tf_n, tf_w, tf_h;
   float tf_scale, grad_scale, iso_n, ert_eps;
   float dscale[3], amb[3], dif[3], spc[3], ldir[3], iso_col[3];
