@@ -242,10 +242,10 @@ struct LeapArgs {
   int nlod, W, H, first, lighting, mode, overlap;
   uint32_t tiles_x;
   // QUEUE_WORDS words cleared before the launch: the grid is persistent and its
-  // waves pull tiles 0 .. ntiles-1 in 8 contiguous chunks, one per XCD
+  // waves pull tiles 0 .. ntiles-1, tile t from the queue of XCD t mod 8
   unsigned int* queues;
   uint32_t ntiles;
-  uint32_t xcd_items[8];        // tiles of each XCD's chunk: ceil(ntiles / 8), the last ones what is left
+  uint32_t xcd_items[8];        // tiles of each XCD's queue
 };
 
 // the 8 contiguous chunks of a persistent launch's n tiles
