@@ -921,20 +921,21 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
             // below); a batch that runs past the phase's end discards the rest.
             // One step body (not unrolled) takes the values in turn, shifted
             // down, so that the shading's registers are not held four times.
-            // The chunked march takes two at a time: four cost it 8-12 spilled
-            // VGPRs (two: 6-10) against 1-4 sampling one at a time.
+            // The chunked march too, although it spills 12 to 16 VGPRs then: three
+            // 1080p frames of the 2048^3 phantom at the 0.25-voxel step took 7.95 ms
+            // two at a time (10 to 14 spilled), 7.25 to 7.5 ms four at a time, 7.8 to
+            // 8.0 ms at two waves without a spill; the fixed march takes 8.0 to 8.2.
             const V3 inc = mk(incTex.x * mlt, incTex.y * mlt, incTex.z * mlt);
-            constexpr int NB = LEARN == 0 ? ISO_BATCH : 2;
-            auto phase = [&](auto fast_c, int end) -> bool {
+                        auto phase = [&](auto fast_c, int end) -> bool {
               while (i < end) {
-                float v[NB];
-                sample_brick_iso_n<T, NB>(bd, nx, ny, nz, edge, pos, inc, v);
-                const int e = min(end, i + NB);
+                float v[ISO_BATCH];
+                sample_brick_iso_n<T>(bd, nx, ny, nz, edge, pos, inc, v);
+                const int e = min(end, i + ISO_BATCH);
 #pragma nounroll
                 for (; i < e; ++i) {
                   if (!step(fast_c, v[0])) return false;
 #pragma unroll
-                  for (int s = 0; s + 1 < NB; ++s) v[s] = v[s + 1];
+                  for (int s = 0; s + 1 < ISO_BATCH; ++s) v[s] = v[s + 1];
                 }
               }
               return true;
@@ -1043,31 +1044,40 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
         const int tn = S.tfst_n;
         const float* __restrict__ ts = S.tfst;
         const float vmaxs = (float)Unorm<T>::max_value();
-        // the lane's chunk at i0: its steps, the transmittance before it, its
-        // value range from the cell grid, the TF statistics over that range
-        // and the contribution bound T0 (1 - (1 - amax)^(s nf))
+        // the lane's chunk at i0: its steps, the transmittance before it and its
+        // value range from the cell grid (range_chunk), the TF statistics over that
+        // range and the contribution bound T0 (1 - (1 - amax)^(s nf)) (bound_chunk)
         int nf = 1, lo = 0, hi = 0;
         float T0 = 0.0f, vl = 0.0f, vh = 0.0f, cnt = 1.0f, amax = 0.0f, smax = 0.0f, obound = 0.0f;
-        auto bound_chunk = [&](int i0) {
+        auto range_chunk = [&](int i0) {
           nf = min(SN_CHUNK, steps - i0);
           T0 = tray * (1.0f - c3);
           uint32_t vlo = 0xffffu, vhi = 0u;
-          // probes at steps 0, pstep, 2 pstep, ... and the chunk's last step
-          for (int q = 0;; q += pstep) {
-            const int qs = min(q, nf - 1);
-            const V3 p = pos + incTex * (float)qs;
-            const float pc[3] = {p.x, p.y, p.z};
-            const int nn3[3] = {nx, ny, nz};
-            int ci[3];
+          // probes at steps 0, pstep, 2 pstep, ... and the chunk's last step, three
+          // at a time with their loads in flight together (the last one again
+          // where fewer are left)
+          for (int q = 0;; q += 3 * pstep) {
+            uint32_t w[3];
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-              const float u = fminf(fmaxf(pc[a], 0.0f), 1.0f) * (float)nn3[a] - 0.5f;
-              ci[a] = min(max((int)floorf(u), 0), nn3[a] - 1) >> CELL_LW;
+            for (int r = 0; r < 3; ++r) {
+              const int qs = min(q + r * pstep, nf - 1);
+              const V3 p = pos + incTex * (float)qs;
+              const float pc[3] = {p.x, p.y, p.z};
+              const int nn3[3] = {nx, ny, nz};
+              int ci[3];
+#pragma unroll
+              for (int a = 0; a < 3; ++a) {
+                const float u = fminf(fmaxf(pc[a], 0.0f), 1.0f) * (float)nn3[a] - 0.5f;
+                ci[a] = min(max((int)floorf(u), 0), nn3[a] - 1) >> CELL_LW;
+              }
+              w[r] = cg[((uint32_t)ci[2] * (uint32_t)ncy + (uint32_t)ci[1]) * (uint32_t)ncx + (uint32_t)ci[0]];
             }
-            const uint32_t w = cg[((uint32_t)ci[2] * (uint32_t)ncy + (uint32_t)ci[1]) * (uint32_t)ncx + (uint32_t)ci[0]];
-            vlo = min(vlo, w & 0xffffu);
-            vhi = max(vhi, w >> 16);
-            if (qs == nf - 1) break;
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+              vlo = min(vlo, w[r] & 0xffffu);
+              vhi = max(vhi, w[r] >> 16);
+            }
+            if (q + 2 * pstep >= nf - 1) break;
           }
           if (border0) vlo = 0u;
           // TF entries of the range (one stored value of slack on either side)
@@ -1079,6 +1089,8 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
           vh = fminf((float)vhi + 1.0f, vmaxs);
           lo = entry_of(vl);
           hi = max(entry_of(vh), lo);
+        };
+        auto bound_chunk = [&]() {
           cnt = (float)(hi - lo + 1);
           const int kk = 31 - __clz(hi - lo + 1);
           amax = fmaxf(ts[tfst_amax(tn, kk) + lo], ts[tfst_amax(tn, kk) + hi - (1 << kk) + 1]);
@@ -1109,9 +1121,18 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
           put(18, obound);
           put(19, T0 * obound);
         };
-        // a skipped chunk: the fixed march's positions, bit for bit
+        // a skipped chunk: the fixed march's positions, bit for bit (eight steps per
+        // turn of the loop: its bookkeeping cost as much as the additions)
         auto skip_steps = [&]() {
-          for (int i = 0; i < nf; ++i) {
+          int i = 0;
+          for (; i + 8 <= nf; i += 8) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+              if (LIT) cur = cur + rayInc;
+              pos = pos + incTex;
+            }
+          }
+          for (; i < nf; ++i) {
             if (LIT) cur = cur + rayInc;
             pos = pos + incTex;
           }
@@ -1127,8 +1148,14 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
           for (;;) {
             bool has = live && i0 < steps;
             while (has) {
-              bound_chunk(i0);
-              if (!(strict && T0 * obound <= LC->skip_bound)) break;
+              range_chunk(i0);
+              // 1D: a range without an opaque entry has amax 0 and the bound 0, told
+              // from the first opaque entry (or the table) without the statistics
+              const bool none = MODE == 0 && (hi < S.tf1_first || (lo > S.tf1_first && (int)S.tf1_next[lo] > hi));
+              if (!(none && strict && 0.0f <= LC->skip_bound)) {
+                bound_chunk();
+                if (!(strict && T0 * obound <= LC->skip_bound)) break;
+              }
               skip_steps();
               i0 += SN_CHUNK;
               has = i0 < steps;
@@ -1174,7 +1201,7 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
           for (int i0 = 0;; i0 += SN_CHUNK) {
             const bool has = live && i0 < steps;
             if (__ballot(has) == 0) break;
-            if (has) bound_chunk(i0);
+            if (has) { range_chunk(i0); bound_chunk(); }
             const bool skip = has && strict && T0 * obound <= LC->skip_bound;
             if (has && !skip) {
               uint32_t h = (uint32_t)(px * 73856093) ^ (uint32_t)(py * 19349663) ^ (fb->toc * 83492791u) ^
