@@ -1365,15 +1365,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TVK_LEARN_W
 }
 
 // Persistent batch launch: every wave pulls tiles from the per-XCD queues until
-// all are drained.  Requests in one launch share MODE, LIT and T.  A cap of 3
-// waves per SIMD lets the lit variants keep their registers (at 4 the lit 2D
-// one spills 2 VGPRs and the learned one 41; measured 44.1 against 44.4 ms on
-// the 64 GiB LOD batch).  Capping only the learned variants at 3 lets the
-// fixed-step ones fit 4 waves with no spill, but that measured slower too
-// (64.5 against 61.6 ms on the 48-request batch, 41.5 against 40.4 ms on the
-// 64 GiB LOD batch).
+// all are drained.  Requests in one launch share MODE, LIT and T.  The fixed-step
+// variants run 4 waves per SIMD, the learned ones (which would spill 41 VGPRs) 3.
+// Batches of 8 requests over 512^3 uint8, 3 waves asked for / 4: lit 2D 12.8 / 12.1
+// and 13.8 / 13.0 ms, unlit 2D 11.5 / 10.9 and 12.7 / 12.0, lit 1D 7.39 / 6.98 and
+// 24.4 / 23.2; unlit 1D and isosurface within 2 % (they fit 4 waves by themselves).
 template <int MODE, bool LIT, typename T, bool COUNT, int LEARN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void batch_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LEARN == 0 ? 4 : 3))) void batch_kernel(
     BatchArgs B, const BatchRequest* __restrict__ req) {
   __shared__ __align__(16) uint16_t s_sn[LEARN > 0 ? 4 * SN_WAVE_LDS : 8];
   __shared__ uint64_t s_cols[MODE == 1 ? 4 * 64 : 1];
