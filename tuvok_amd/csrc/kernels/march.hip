@@ -1053,13 +1053,13 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
           nf = min(SN_CHUNK, steps - i0);
           T0 = tray * (1.0f - c3);
           uint32_t vlo = 0xffffu, vhi = 0u;
-          // probes at steps 0, pstep, 2 pstep, ... and the chunk's last step, three
+          // probes at steps 0, pstep, 2 pstep, ... and the chunk's last step, four
           // at a time with their loads in flight together (the last one again
           // where fewer are left)
-          for (int q = 0;; q += 3 * pstep) {
-            uint32_t w[3];
+                    for (int q = 0;; q += 4 * pstep) {
+            uint32_t w[4];
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
+            for (int r = 0; r < 4; ++r) {
               const int qs = min(q + r * pstep, nf - 1);
               const V3 p = pos + incTex * (float)qs;
               const float pc[3] = {p.x, p.y, p.z};
@@ -1073,11 +1073,11 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
               w[r] = cg[((uint32_t)ci[2] * (uint32_t)ncy + (uint32_t)ci[1]) * (uint32_t)ncx + (uint32_t)ci[0]];
             }
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
+            for (int r = 0; r < 4; ++r) {
               vlo = min(vlo, w[r] & 0xffffu);
               vhi = max(vhi, w[r] >> 16);
             }
-            if (q + 2 * pstep >= nf - 1) break;
+            if (q + 3 * pstep >= nf - 1) break;
           }
           if (border0) vlo = 0u;
           // TF entries of the range (one stored value of slack on either side)
@@ -1149,9 +1149,9 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
             bool has = live && i0 < steps;
             while (has) {
               range_chunk(i0);
-              // 1D: a range without an opaque entry has amax 0 and the bound 0, told
-              // from the first opaque entry (or the table) without the statistics
-              const bool none = MODE == 0 && (hi < S.tf1_first || (lo > S.tf1_first && (int)S.tf1_next[lo] > hi));
+              // 1D: a range below the first opaque entry has amax 0 and the bound 0,
+              // without the statistics
+              const bool none = MODE == 0 && hi < S.tf1_first;
               if (!(none && strict && 0.0f <= LC->skip_bound)) {
                 bound_chunk();
                 if (!(strict && T0 * obound <= LC->skip_bound)) break;
