@@ -316,8 +316,8 @@ int tvk_batch_create(tvk_batch** out, int device) {
   tvk_default_tuning(&b->tune);
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_queues, QUEUE_WORDS * sizeof(unsigned int));
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_counter, sizeof(unsigned long long));
+  if (e == hipSuccess) e = device_alloc(&b->d_queues, QUEUE_WORDS * sizeof(unsigned int));
+  if (e == hipSuccess) e = device_alloc(&b->d_counter, sizeof(unsigned long long));
   if (e == hipSuccess) e = hipEventCreate(&b->ev[0]);
   if (e == hipSuccess) e = hipEventCreate(&b->ev[1]);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&b->cu_count, hipDeviceAttributeMultiprocessorCount, device);

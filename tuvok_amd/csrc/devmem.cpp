@@ -1,5 +1,6 @@
 #include "devmem.hpp"
 #include <algorithm>
+#include <cstdint>
 #include <map>
 #include <mutex>
 #include <new>
@@ -16,6 +17,7 @@ struct Kept {
   std::vector<Block> blocks;   // the longest kept first
   size_t bytes = 0, limit = 0;
   int users = 0;
+  uint64_t trims = 0;          // how often the blocks were freed
 };
 constexpr size_t kMaxBlocks = 16;
 
@@ -32,6 +34,7 @@ bool trim(Kept& k) {
   for (const Block& b : k.blocks) (void)hipFree(b.p);
   k.blocks.clear();
   k.bytes = 0;
+  ++k.trims;
   return true;
 }
 
@@ -64,16 +67,26 @@ void give_back(int device, void* p, size_t bytes) {
 }  // namespace
 
 hipError_t device_alloc_bytes(void** p, size_t bytes) {
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipErrorOutOfMemory) return e;
   int device = 0;
-  if (hipGetDevice(&device) != hipSuccess) return e;
+  hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
+  uint64_t seen;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (!trim(kept()[device])) return e;
+    seen = kept()[device].trims;
   }
-  (void)hipGetLastError();
-  return hipMalloc(p, bytes);
+  for (;;) {
+    e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    {
+      std::lock_guard<std::mutex> lk(g_mu);
+      Kept& k = kept()[device];
+      // nothing to free now, nor freed by another thread since this one last tried
+      if (!trim(k) && k.trims == seen) return e;
+      seen = k.trims;
+    }
+    (void)hipGetLastError();
+  }
 }
 
 hipError_t device_block(std::shared_ptr<void>* out, size_t bytes) {
