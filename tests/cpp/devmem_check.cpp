@@ -83,7 +83,30 @@ static int two_threads_out_of_memory() {
   return 0;
 }
 
+// A block that does not fit takes the room of one the caller can do without, and
+// leaves it alone where there is room.
+static int spare_block() {
+  device_hold(0);
+  {
+    void* rest = nullptr;
+    std::shared_ptr<void> spare, a, b;
+    CHECK(device_block(&spare, 70 * MB) == hipSuccess);   // larger than what may be kept
+    CHECK(hipMalloc(&rest, 904 * MB) == hipSuccess);   // 50 MiB are free
+    CHECK(device_block(&a, 10 * MB, &spare) == hipSuccess && spare);
+    CHECK(device_block(&b, 100 * MB, &spare) == hipSuccess && !spare);
+    std::shared_ptr<void> c;
+    CHECK(device_block(&c, 100 * MB, &spare) == hipErrorOutOfMemory && !c);
+    CHECK(device_block(&spare, 5 * MB) == hipSuccess);
+    CHECK(device_block(&c, 8 * MB, &spare) == hipSuccess && !spare);   // 10 MiB with the spare's, which was kept
+    CHECK(hipFree(rest) == hipSuccess);
+  }
+  device_drop(0);
+  CHECK(used == 0);
+  return 0;
+}
+
 int main() {
+  if (spare_block()) return 1;
   if (two_threads_out_of_memory()) return 1;
   std::printf("ok\n");
   return 0;

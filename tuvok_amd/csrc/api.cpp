@@ -46,35 +46,33 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
   HIPCHK(c, device_block(&c->pool_hold, c->pool_bytes));
   c->d_pool = c->pool_hold.get();
   c->cells = std::make_shared<CellGrid>();
-  // descriptors of every kept brick
-  std::vector<GatherBrick> gb(L.toc.size());
-  for (size_t i = 0; i < L.toc.size(); ++i) {
-    for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)L.toc[i].coords[k]; gb[i].n[k] = L.toc[i].size[k]; }
-    gb[i].offset = L.toc[i].offset;
+  // descriptors of every kept brick and their first cells, behind them the
+  // per-brick min/max: folded into the gather; recomputed for the levels whose
+  // overlaps FillOverlap rewrites afterwards
+  CellTables tab;
+  cell_tables(L, tab);
+  std::shared_ptr<void> tab_hold, quad_hold, words_hold, snap_hold, tmp[2];
+  HIPCHK(c, device_block(&tab_hold, tab.host.size() + 2 * L.toc.size() * sizeof(uint32_t)));
+  const GatherBrick* const d_gb = (const GatherBrick*)tab_hold.get();
+  uint32_t* const d_mm = (uint32_t*)((uint8_t*)tab_hold.get() + tab.host.size());
+  HIPCHK(c, hipMemcpyAsync(tab_hold.get(), tab.host.data(), tab.host.size(), hipMemcpyHostToDevice, c->stream));
+  // the cell grid's words and the ranges of every 4^3 voxels, written with the
+  // bricks.  Where memory is short the bricks go first: the ranges and the words are
+  // given up for the blocks below, and the grid is made on first use instead.
+  auto block = [&](std::shared_ptr<void>* h, size_t bytes) {
+    const hipError_t e = device_block(h, bytes, &quad_hold);
+    return e == hipErrorOutOfMemory && words_hold ? device_block(h, bytes, &words_hold) : e;
+  };
+  if (tab.total < (1ull << 32)) {
+    (void)device_block(&quad_hold, quad_words(L) * sizeof(uint32_t));
+    if (quad_hold) (void)device_block(&words_hold, std::max<uint64_t>(tab.total, 1) * sizeof(uint32_t), &quad_hold);
+    if (!quad_hold || !words_hold) { (void)hipGetLastError(); quad_hold.reset(); words_hold.reset(); }
   }
-  std::shared_ptr<void> gb_hold, mm_hold, snap_hold, tmp[2];
-  HIPCHK(c, device_block(&gb_hold, gb.size() * sizeof(GatherBrick)));
-  GatherBrick* d_gb = (GatherBrick*)gb_hold.get();
-  HIPCHK(c, hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream));
   const void* src = d_lin;
   int rc = TVK_OK;
   hipEvent_t ev[2] = {nullptr, nullptr};
   if (hipEventCreate(&ev[0]) != hipSuccess || hipEventCreate(&ev[1]) != hipSuccess) ev[0] = ev[1] = nullptr;
   if (ev[0]) (void)hipEventRecord(ev[0], c->stream);
-  // per-brick min/max: folded into the gather; recomputed for the levels whose
-  // overlaps FillOverlap rewrites afterwards
-  uint32_t* d_mm = nullptr;
-  {
-    hipError_t e = device_block(&mm_hold, 2 * gb.size() * sizeof(uint32_t));
-    if (e != hipSuccess) rc = hipfail(c, "hipMalloc(minmax)", e);
-    d_mm = (uint32_t*)mm_hold.get();
-  }
-  // ranges of every 4^3 voxels, written with the bricks (without room for them
-  // the cell grid is made on first use instead)
-  std::shared_ptr<void> quad_hold;
-  (void)device_block(&quad_hold, quad_words(L) * sizeof(uint32_t));
-  if (!quad_hold) (void)hipGetLastError();
-  uint32_t* const d_quads = (uint32_t*)quad_hold.get();
   bool refilled = false;
   void* d_snap = nullptr;   // a level's bricks before FillOverlap (odd cores)
   for (size_t lod = 0; lod < keep && rc == TVK_OK; ++lod) {
@@ -100,7 +98,7 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
         std::shared_ptr<void>& hold = tmp[(lod - 1) % 2];
         if (!hold) {
           size_t bytes = (size_t)(li.size[0] * li.size[1] * li.size[2]) * bpv;
-          hipError_t e = device_block(&hold, bytes);
+          hipError_t e = block(&hold, bytes);
           if (e != hipSuccess) { rc = hipfail(c, "hipMalloc(lod temp)", e); break; }
         }
         void* const dst = hold.get();
@@ -109,7 +107,7 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
         src = dst;
       }
       hipError_t e = launch_gather(src, bpv, li.size, d_gb + li.offset, nb, (uint32_t)li.bricks[0], maxv, c->d_pool,
-                                   core, L.overlap, c->clamp, d_mm + 2 * li.offset, d_quads, c->stream);
+                                   core, L.overlap, c->clamp, d_mm + 2 * li.offset, (uint32_t*)quad_hold.get(), c->stream);
       if (e != hipSuccess) { rc = hipfail(c, "gather", e); break; }
     }
     if (lod > 0 && !c->clamp && nb > 1) {
@@ -121,7 +119,7 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
         snap_base = L.toc[li.offset].offset;
         const size_t bytes = (size_t)(last.offset + last.count - snap_base) * bpv;
         snap_hold.reset();
-        e = device_block(&snap_hold, bytes);
+        e = block(&snap_hold, bytes);
         d_snap = snap_hold.get();
         if (e == hipSuccess)
           e = hipMemcpyAsync(d_snap, (uint8_t*)c->d_pool + snap_base * bpv, bytes, hipMemcpyDeviceToDevice,
@@ -143,7 +141,7 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
       }
       start.push_back((uint32_t)order.size());
       std::shared_ptr<void> order_hold;
-      if (e == hipSuccess) e = device_block(&order_hold, order.size() * sizeof(uint32_t));
+      if (e == hipSuccess) e = block(&order_hold, order.size() * sizeof(uint32_t));
       uint32_t* const d_order = (uint32_t*)order_hold.get();
       if (e == hipSuccess)
         e = hipMemcpyAsync(d_order, order.data(), order.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
@@ -167,14 +165,18 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
     const size_t first = L.lods[1].offset;
     uint32_t maxv = 0;
     for (size_t i = first; i < L.toc.size(); ++i) maxv = std::max<uint32_t>(maxv, (uint32_t)L.toc[i].count);
-    hipError_t e = launch_extend(c->d_pool, bpv, d_gb + first, (uint32_t)(gb.size() - first), maxv, c->stream);
+    hipError_t e = launch_extend(c->d_pool, bpv, d_gb + first, (uint32_t)(L.toc.size() - first), maxv, c->stream);
     if (e == hipSuccess)
-      e = launch_minmax(c->d_pool, bpv, d_gb + first, (uint32_t)(gb.size() - first), maxv, d_mm + 2 * first, d_quads,
-                        c->stream);
+      e = launch_minmax(c->d_pool, bpv, d_gb + first, (uint32_t)(L.toc.size() - first), maxv, d_mm + 2 * first,
+                        (uint32_t*)quad_hold.get(), c->stream);
     if (e != hipSuccess) rc = hipfail(c, "extend/minmax", e);
   }
   if (ev[1]) (void)hipEventRecord(ev[1], c->stream);
-  std::vector<uint32_t> mm(2 * gb.size());
+  // a grid that could not be launched is made on first use
+  const bool cells = rc == TVK_OK && quad_hold && words_hold &&
+                     launch_cells((const uint32_t*)quad_hold.get(), bpv, d_gb, tab.base_of(d_gb),
+                                  (uint32_t)L.toc.size(), tab.max_cells, (uint32_t*)words_hold.get(), c->stream) == hipSuccess;
+  std::vector<uint32_t> mm(2 * L.toc.size());
   if (rc == TVK_OK) {
     hipError_t e = hipMemcpyAsync(mm.data(), d_mm, mm.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -186,10 +188,9 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
   for (hipEvent_t e : ev)
     if (e) (void)hipEventDestroy(e);
   if (rc != TVK_OK) return rc;
-  if (d_quads) {
-    const std::string msg = c->err;
+  if (cells) {
     std::lock_guard<std::mutex> lk(c->cells->mu);
-    if (make_cells(c, *c->cells, d_quads) != TVK_OK) { (void)hipGetLastError(); c->err = msg; }   // marches go without it
+    publish_cells(*c->cells, std::move(words_hold), std::move(tab.base));
   }
   c->minmax.resize(mm.size());
   for (size_t i = 0; i < mm.size(); ++i) c->minmax[i] = (double)mm[i];
@@ -1143,95 +1144,106 @@ int learn_prepare(tvk_ctx* c) {
   return ensure_cells(c);
 }
 
-int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads) {
-  const Layout& L = c->L;
-  std::vector<GatherBrick> gb(L.toc.size());
-  uint32_t* words = G.words.load(std::memory_order_relaxed);
-  if (!words) G.base.assign(L.toc.size(), 0);   // no other thread reads it yet
-  uint64_t total = 0;
-  uint32_t max_cells = 0, max_vox = 0;
-  for (size_t i = 0; i < L.toc.size(); ++i) {
-    for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)L.toc[i].coords[k]; gb[i].n[k] = L.toc[i].size[k]; }
-    gb[i].offset = L.toc[i].offset;
-    const uint32_t nc = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
-    if (!words) G.base[i] = (uint32_t)total;
-    total += nc;
-    max_cells = std::max(max_cells, nc);
-    max_vox = std::max(max_vox, (uint32_t)L.toc[i].count);
+void cell_tables(const Layout& L, CellTables& T) {
+  const size_t n = L.toc.size();
+  T = CellTables{};
+  T.n = n;
+  T.base.resize(n);
+  T.host.resize(n * (sizeof(GatherBrick) + sizeof(uint32_t)));
+  for (size_t i = 0; i < n; ++i) {
+    GatherBrick g;
+    for (int k = 0; k < 3; ++k) { g.c[k] = (uint32_t)L.toc[i].coords[k]; g.n[k] = L.toc[i].size[k]; }
+    g.offset = L.toc[i].offset;
+    std::memcpy(T.host.data() + i * sizeof(g), &g, sizeof(g));
+    const uint32_t nc = cell_count(g.n[0]) * cell_count(g.n[1]) * cell_count(g.n[2]);
+    T.base[i] = (uint32_t)T.total;
+    T.total += nc;
+    T.max_cells = std::max(T.max_cells, nc);
+    T.max_vox = std::max(T.max_vox, (uint32_t)L.toc[i].count);
   }
-  if (total >= (1ull << 32)) return fail(c, TVK_ERR_UNSUPPORTED, "cell grid exceeds 2^32 cells");
-  std::shared_ptr<void> gb_hold, base_hold, quad_hold;
-  hipError_t e = hipSuccess;
-  if (!G.hold) e = device_block(&G.hold, std::max<uint64_t>(total, 1) * sizeof(uint32_t));
-  words = (uint32_t*)G.hold.get();
-  if (e == hipSuccess) e = device_block(&gb_hold, gb.size() * sizeof(GatherBrick));
-  if (e == hipSuccess) e = device_block(&base_hold, G.base.size() * sizeof(uint32_t));
-  if (e == hipSuccess && !quads) e = device_block(&quad_hold, quad_words(L) * sizeof(uint32_t));
-  if (e != hipSuccess) return hipfail(c, "cell grid", e);
-  GatherBrick* const d_gb = (GatherBrick*)gb_hold.get();
-  e = hipMemcpyAsync(d_gb, gb.data(), gb.size() * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(base_hold.get(), G.base.data(), G.base.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess && !quads) {
-    e = launch_minmax(c->d_pool, L.bpv, d_gb, (uint32_t)gb.size(), max_vox, nullptr, (uint32_t*)quad_hold.get(), c->stream);
-    quads = (const uint32_t*)quad_hold.get();
-  }
-  if (e == hipSuccess)
-    e = launch_cells(quads, L.bpv, d_gb, (const uint32_t*)base_hold.get(), (uint32_t)gb.size(), max_cells,
-                     words, c->stream);
-  const hipError_t se = hipStreamSynchronize(c->stream);
-  if (e == hipSuccess) e = se;
-  if (e != hipSuccess) return hipfail(c, "cell grid", e);
-  G.words.store(words, std::memory_order_release);
-  G.stale.assign(L.toc.size(), 0);
-  G.ready.store(true, std::memory_order_release);
-  return TVK_OK;
+  std::memcpy(T.host.data() + n * sizeof(GatherBrick), T.base.data(), n * sizeof(uint32_t));
 }
 
-int remake_cells(tvk_ctx* c, CellGrid& G) {
+void publish_cells(CellGrid& G, std::shared_ptr<void> words, std::vector<uint32_t> base) {
+  G.stale.assign(base.size(), 0);
+  G.base = std::move(base);
+  G.hold = std::move(words);
+  G.words.store((uint32_t*)G.hold.get(), std::memory_order_release);
+  G.ready.store(true, std::memory_order_release);
+}
+
+// The words of the listed bricks, one brick at a time through the grid's own buffer
+// (descriptors, first cells, and the ranges of 4^3 voxels of the largest brick).
+static hipError_t cells_by_brick(tvk_ctx* c, CellGrid& G, const CellTables& tab, const std::vector<uint32_t>& list,
+                                 uint32_t* words) {
   const Layout& L = c->L;
-  std::vector<uint32_t> list;
-  for (uint32_t t = 0; t < L.toc.size(); ++t)
-    if (G.stale[t]) list.push_back(t);
-  const size_t n = list.size();
-  if (8 * n >= L.toc.size()) return make_cells(c, G, nullptr);
-  // one brick at a time through a quad buffer of the largest
   const uint32_t per = L.bpv == 1 ? 256u : 128u, h = L.bpv == 1 ? 2u : 1u;   // elements and quads of a block
-  std::vector<GatherBrick> gb(n);
-  std::vector<uint32_t> base(n);
-  uint64_t most = 0;
-  for (size_t i = 0; i < n; ++i) {
-    const TocBrick& t = L.toc[list[i]];
-    for (int k = 0; k < 3; ++k) { gb[i].c[k] = (uint32_t)t.coords[k]; gb[i].n[k] = t.size[k]; }
-    gb[i].offset = t.offset;
-    base[i] = G.base[list[i]];
-    most = std::max<uint64_t>(most, t.count);
+  const size_t quads_at = (tab.host.size() + 255) & ~(size_t)255;
+  if (!G.scratch) {
+    hipError_t e = device_block(&G.scratch, quads_at + (size_t)(tab.max_vox / per) * h * sizeof(uint32_t));
+    if (e != hipSuccess) return e;
+    e = hipMemcpyAsync(G.scratch.get(), tab.host.data(), tab.host.size(), hipMemcpyHostToDevice, c->stream);
+    if (e != hipSuccess) { (void)hipStreamSynchronize(c->stream); G.scratch.reset(); return e; }
   }
-  std::shared_ptr<void> gb_hold, base_hold, quad_hold;
-  hipError_t e = device_block(&gb_hold, n * sizeof(GatherBrick));
-  if (e == hipSuccess) e = device_block(&base_hold, n * sizeof(uint32_t));
-  if (e == hipSuccess) e = device_block(&quad_hold, (size_t)(most / per) * h * sizeof(uint32_t));
-  if (e != hipSuccess) return hipfail(c, "cell grid", e);
-  const GatherBrick* const d_gb = (const GatherBrick*)gb_hold.get();
-  e = hipMemcpyAsync(gb_hold.get(), gb.data(), n * sizeof(GatherBrick), hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(base_hold.get(), base.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream);
-  for (size_t i = 0; i < n && e == hipSuccess; ++i) {
+  const GatherBrick* const d_gb = (const GatherBrick*)G.scratch.get();
+  const uint32_t* const d_base = tab.base_of(d_gb);
+  hipError_t e = hipSuccess;
+  for (size_t i = 0; i < list.size() && e == hipSuccess; ++i) {
+    const TocBrick& t = L.toc[list[i]];
     // the kernels index quads by the brick's place in the pool: the buffer
     // stands where that brick's quads would be
-    const uintptr_t shift = (uintptr_t)(gb[i].offset / per) * h * sizeof(uint32_t);
-    uint32_t* const quads = (uint32_t*)((uintptr_t)quad_hold.get() - shift);
-    const uint32_t cells = cell_count(gb[i].n[0]) * cell_count(gb[i].n[1]) * cell_count(gb[i].n[2]);
-    e = launch_minmax(c->d_pool, L.bpv, d_gb + i, 1, (uint32_t)L.toc[list[i]].count, nullptr, quads, c->stream);
-    if (e == hipSuccess)
-      e = launch_cells(quads, L.bpv, d_gb + i, (const uint32_t*)base_hold.get() + i, 1, cells,
-                       G.words.load(std::memory_order_relaxed), c->stream);
+    const uintptr_t shift = (uintptr_t)(t.offset / per) * h * sizeof(uint32_t);
+    uint32_t* const quads = (uint32_t*)((uintptr_t)G.scratch.get() + quads_at - shift);
+    const uint32_t cells = cell_count(t.size[0]) * cell_count(t.size[1]) * cell_count(t.size[2]);
+    e = launch_minmax(c->d_pool, L.bpv, d_gb + list[i], 1, (uint32_t)t.count, nullptr, quads, c->stream);
+    if (e == hipSuccess) e = launch_cells(quads, L.bpv, d_gb + list[i], d_base + list[i], 1, cells, words, c->stream);
+  }
+  return e;
+}
+
+// The words of every brick (none made yet) or of the stale ones; needs G.mu.  From
+// an eighth of the bricks on, and more than 16, all of them at once: two launches
+// instead of two per brick, through blocks that go back, and with room for them.
+static int make_cells(tvk_ctx* c, CellGrid& G) {
+  const Layout& L = c->L;
+  CellTables tab;
+  cell_tables(L, tab);
+  if (tab.total >= (1ull << 32)) return fail(c, TVK_ERR_UNSUPPORTED, "cell grid exceeds 2^32 cells");
+  uint32_t* words = G.words.load(std::memory_order_relaxed);
+  std::vector<uint32_t> list;
+  for (uint32_t t = 0; t < L.toc.size(); ++t)
+    if (!words || G.stale[t]) list.push_back(t);
+  std::shared_ptr<void> words_hold, tab_hold, quad_hold;
+  hipError_t e = hipSuccess;
+  if (!words) {
+    e = device_block(&words_hold, std::max<uint64_t>(tab.total, 1) * sizeof(uint32_t));
+    if (e != hipSuccess) return hipfail(c, "cell grid", e);
+  }
+  uint32_t* const out = words ? words : (uint32_t*)words_hold.get();
+  if (list.size() > 16 && 8 * list.size() >= L.toc.size()) {
+    (void)device_block(&tab_hold, tab.host.size());
+    if (tab_hold) (void)device_block(&quad_hold, quad_words(L) * sizeof(uint32_t));
+    if (!quad_hold) (void)hipGetLastError();
+  }
+  if (quad_hold) {
+    const GatherBrick* const d_gb = (const GatherBrick*)tab_hold.get();
+    uint32_t* const quads = (uint32_t*)quad_hold.get();
+    const uint32_t n = (uint32_t)L.toc.size();
+    e = hipMemcpyAsync(tab_hold.get(), tab.host.data(), tab.host.size(), hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = launch_minmax(c->d_pool, L.bpv, d_gb, n, tab.max_vox, nullptr, quads, c->stream);
+    if (e == hipSuccess) e = launch_cells(quads, L.bpv, d_gb, tab.base_of(d_gb), n, tab.max_cells, out, c->stream);
+  } else {
+    e = cells_by_brick(c, G, tab, list, out);
   }
   const hipError_t se = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) e = se;
   if (e != hipSuccess) return hipfail(c, "cell grid", e);
-  G.stale.assign(L.toc.size(), 0);
-  G.ready.store(true, std::memory_order_release);
+  if (words) {
+    G.stale.assign(L.toc.size(), 0);
+    G.ready.store(true, std::memory_order_release);
+  } else {
+    publish_cells(G, std::move(words_hold), std::move(tab.base));
+  }
   return TVK_OK;
 }
 
@@ -1242,8 +1254,7 @@ int ensure_cells(tvk_ctx* c) {
   CellGrid& G = *c->cells;
   if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
   std::lock_guard<std::mutex> lk(G.mu);
-  if (G.ready.load(std::memory_order_acquire)) return TVK_OK;
-  return G.words.load(std::memory_order_relaxed) ? remake_cells(c, G) : make_cells(c, G, nullptr);
+  return G.ready.load(std::memory_order_acquire) ? TVK_OK : make_cells(c, G);
 }
 
 void brick_tf_stats(tvk_ctx* c, FrameBrick& fb) {

@@ -98,15 +98,25 @@ struct PoolState {
 // the contexts that share the dataset, whatever thread each is used on.  What a
 // render holds on to never moves: `words` is set once and `base`, which the layout
 // alone decides, is filled before that.  A brick uploaded again clears `ready` for
-// all of them; the next use makes that brick's words again in place (an eighth
-// of the bricks or more: all of them).
+// all of them; the next use makes that brick's words again in place.
 struct CellGrid {
   std::mutex mu;                // held while the words are made, and for stale
   std::atomic<bool> ready{false};   // the words are those of the bricks as they are
   std::atomic<uint32_t*> words{nullptr};
   std::vector<uint32_t> base;   // first cell of each TOC brick (read where words is set)
   std::vector<uint8_t> stale;   // per TOC brick: uploaded again since the words were made
-  std::shared_ptr<void> hold;
+  std::shared_ptr<void> hold;   // owns words
+  std::shared_ptr<void> scratch;   // of making single bricks' words again (no block goes back, no wait for the device)
+};
+// What the kernels that make the words need of every TOC brick: descriptors and,
+// behind them, the first cells, as they are uploaded together.
+struct CellTables {
+  size_t n = 0;
+  std::vector<uint8_t> host;
+  std::vector<uint32_t> base;
+  uint64_t total = 0;           // cells
+  uint32_t max_cells = 0, max_vox = 0;   // of a brick (max_vox: its padded elements)
+  const uint32_t* base_of(const GatherBrick* d) const { return (const uint32_t*)(d + n); }
 };
 }  // namespace tvk
 
@@ -312,11 +322,9 @@ void brick_tf_stats(tvk_ctx* c, FrameBrick& fb);
 int learn_prepare(tvk_ctx* c);
 // the dataset's cell grid (made on first use)
 int ensure_cells(tvk_ctx* c);
-// The cell grid from quad ranges of every brick (quads, or null: read from the
-// pool), stream-ordered; needs G.mu.
-int make_cells(tvk_ctx* c, CellGrid& G, const uint32_t* quads);
-// The words of the stale bricks alone; needs G.mu and a grid made before.
-int remake_cells(tvk_ctx* c, CellGrid& G);
+void cell_tables(const Layout& L, CellTables& T);
+// Words made for the first time are the grid's from here on; needs G.mu.
+void publish_cells(CellGrid& G, std::shared_ptr<void> words, std::vector<uint32_t> base);
 inline size_t quad_words(const Layout& L) { return (size_t)(L.pool_elems / (L.bpv == 1 ? 256u : 128u)) * (L.bpv == 1 ? 2u : 1u); }
 // the cell grid as the kernels read it; null while it is not made, for
 // compatibility textures and for a budgeted pool

@@ -89,7 +89,7 @@ hipError_t device_alloc_bytes(void** p, size_t bytes) {
   }
 }
 
-hipError_t device_block(std::shared_ptr<void>* out, size_t bytes) {
+hipError_t device_block(std::shared_ptr<void>* out, size_t bytes, std::shared_ptr<void>* spare) {
   out->reset();
   int device = 0;
   hipError_t e = hipGetDevice(&device);
@@ -114,6 +114,11 @@ hipError_t device_block(std::shared_ptr<void>* out, size_t bytes) {
   }
   if (!p) {
     e = device_alloc_bytes(&p, want);
+    if (e == hipErrorOutOfMemory && spare && *spare) {
+      (void)hipGetLastError();
+      spare->reset();   // kept, and freed by the next attempt
+      e = device_alloc_bytes(&p, want);
+    }
     if (e != hipSuccess) return e;
   }
   *out = std::shared_ptr<void>(p, [device, want](void* q) { give_back(device, q, want); });

@@ -24,8 +24,9 @@ template <typename T>
 hipError_t device_alloc(T** p, size_t bytes) { return device_alloc_bytes(reinterpret_cast<void**>(p), bytes); }
 
 // A block of at least `bytes` on the current device, a kept one or a new one; it
-// goes back with its last reference.  Contents are undefined.
-hipError_t device_block(std::shared_ptr<void>* out, size_t bytes);
+// goes back with its last reference.  Contents are undefined.  spare: a block the
+// caller can do without; it is given up (left null) where there is no room else.
+hipError_t device_block(std::shared_ptr<void>* out, size_t bytes, std::shared_ptr<void>* spare = nullptr);
 
 // contexts of a device: the last one to go gives back what is kept
 void device_hold(int device);
