@@ -5,8 +5,9 @@ using namespace tvk;
 
 namespace {
 
-std::vector<float4> unorm_table(const uint8_t* rgba8, size_t n) {
-  std::vector<float4> f(n);
+// more: entries behind the table's, zeros
+std::vector<float4> unorm_table(const uint8_t* rgba8, size_t n, size_t more = 0) {
+  std::vector<float4> f(n + more);
   for (size_t i = 0; i < n; ++i)
     f[i] = make_float4((float)rgba8[4 * i] / 255.0f, (float)rgba8[4 * i + 1] / 255.0f,
                        (float)rgba8[4 * i + 2] / 255.0f, (float)rgba8[4 * i + 3] / 255.0f);
@@ -182,7 +183,8 @@ int build_pool(tvk_ctx* c, const void* d_lin) {
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) rc = hipfail(c, "minmax download", e);
   }
-  (void)hipStreamSynchronize(c->stream);
+  if (hipStreamSynchronize(c->stream) == hipSuccess)
+    for (const auto& h : {tab_hold, quad_hold, snap_hold, tmp[0], tmp[1]}) device_idle(h);
   c->build_ms = 0.0f;
   if (ev[0] && ev[1] && rc == TVK_OK) (void)hipEventElapsedTime(&c->build_ms, ev[0], ev[1]);
   for (hipEvent_t e : ev)
@@ -371,7 +373,7 @@ int tvk_load_volume(tvk_ctx* c, const void* host, int dtype, const uint64_t dims
   HIPCHK(c, hipMemcpyAsync(c->d_lin, host, bytes, hipMemcpyHostToDevice, c->stream));
   rc = build_pool(c, c->d_lin);
   if (!keep_linear || rc) {
-    (void)hipStreamSynchronize(c->stream);
+    if (hipStreamSynchronize(c->stream) == hipSuccess) device_idle(c->lin_hold);
     c->lin_hold.reset();
     c->d_lin = nullptr;
     c->lin_bytes = 0;
@@ -459,7 +461,7 @@ int tvk_generate_volume(tvk_ctx* c, int kind, uint64_t seed, int dtype, const ui
   if (e != hipSuccess) { free_dataset(c); return hipfail(c, "generate", e); }
   rc = build_pool(c, c->d_lin);
   if (!keep_linear || rc) {
-    (void)hipStreamSynchronize(c->stream);
+    if (hipStreamSynchronize(c->stream) == hipSuccess) device_idle(c->lin_hold);
     c->lin_hold.reset();
     c->d_lin = nullptr;
     c->lin_bytes = 0;
@@ -722,7 +724,8 @@ int download_ref(tvk_ctx* c, size_t first, size_t n, void* host, size_t bytes) {
   if (e == hipSuccess) e = launch_unswizzle(c->d_pool, L.bpv, d_gb, d_ro, (uint32_t)n, maxv, d_out, c->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(host, d_out, bytes, hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  (void)hipStreamSynchronize(c->stream);
+  if (hipStreamSynchronize(c->stream) == hipSuccess)
+    for (const auto& h : {gb_hold, ro_hold, out_hold}) device_idle(h);
   if (e != hipSuccess) return hipfail(c, "brick download", e);
   return TVK_OK;
 }
@@ -790,6 +793,8 @@ int tvk_max_gradient(tvk_ctx* c, float* out) {
       HIPCHK(c, hipStreamSynchronize(c->stream));
       for (size_t k = 0; k < (size_t)cnt * gx; ++k) m = std::max(m, h[k]);
     }
+    device_idle(gb_hold);   // the stream was waited for
+    device_idle(part_hold);
     *out = (float)m;
     return TVK_OK;
   }
@@ -1238,6 +1243,8 @@ static int make_cells(tvk_ctx* c, CellGrid& G) {
   const hipError_t se = hipStreamSynchronize(c->stream);
   if (e == hipSuccess) e = se;
   if (e != hipSuccess) return hipfail(c, "cell grid", e);
+  device_idle(tab_hold);
+  device_idle(quad_hold);
   if (words) {
     G.stale.assign(L.toc.size(), 0);
     G.ready.store(true, std::memory_order_release);

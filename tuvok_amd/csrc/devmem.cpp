@@ -38,12 +38,12 @@ bool trim(Kept& k) {
   return true;
 }
 
-void give_back(int device, void* p, size_t bytes) {
+void give_back(int device, void* p, size_t bytes, bool idle) {
   int cur = device;
   (void)hipGetDevice(&cur);
   if (cur != device) (void)hipSetDevice(device);
   bool keep = false;
-  if (hipDeviceSynchronize() == hipSuccess) {
+  if (idle || hipDeviceSynchronize() == hipSuccess) {
     std::lock_guard<std::mutex> lk(g_mu);
     Kept& k = kept()[device];
     if (k.users > 0 && bytes <= k.limit) {
@@ -63,6 +63,13 @@ void give_back(int device, void* p, size_t bytes) {
   if (!keep) (void)hipFree(p);
   if (cur != device) (void)hipSetDevice(cur);
 }
+
+struct GiveBack {
+  int device;
+  size_t bytes;
+  bool idle = false;
+  void operator()(void* p) const { give_back(device, p, bytes, idle); }
+};
 
 }  // namespace
 
@@ -121,8 +128,12 @@ hipError_t device_block(std::shared_ptr<void>* out, size_t bytes, std::shared_pt
     }
     if (e != hipSuccess) return e;
   }
-  *out = std::shared_ptr<void>(p, [device, want](void* q) { give_back(device, q, want); });
+  *out = std::shared_ptr<void>(p, GiveBack{device, want});
   return hipSuccess;
+}
+
+void device_idle(const std::shared_ptr<void>& block) {
+  if (GiveBack* g = std::get_deleter<GiveBack>(block)) g->idle = true;
 }
 
 void device_hold(int device) {

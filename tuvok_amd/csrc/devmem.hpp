@@ -10,7 +10,8 @@
 // the longest kept go first) and given back: when an allocation fails
 // (device_alloc frees what is kept and tries again) and when the device's last
 // context is destroyed.  A block is kept only after hipDeviceSynchronize, which
-// hipFree implies too, so no queued work still uses it, whatever the stream.
+// hipFree implies too, so no queued work still uses it, whatever the stream; a
+// caller that has waited for the only stream that used it says so (device_idle).
 // All calls are safe from several threads.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -27,6 +28,10 @@ hipError_t device_alloc(T** p, size_t bytes) { return device_alloc_bytes(reinter
 // goes back with its last reference.  Contents are undefined.  spare: a block the
 // caller can do without; it is given up (left null) where there is no room else.
 hipError_t device_block(std::shared_ptr<void>* out, size_t bytes, std::shared_ptr<void>* spare = nullptr);
+
+// Says that no queued work uses the block any more (its stream was waited for, and
+// no other saw it): it goes back without a wait for the whole device.
+void device_idle(const std::shared_ptr<void>& block);
 
 // contexts of a device: the last one to go gives back what is kept
 void device_hold(int device);
