@@ -336,7 +336,6 @@ void tvk_destroy(tvk_ctx* c) {
   for (void* q : {(void*)c->d_leap_meta, (void*)c->d_leap_table, (void*)c->d_leap_bricks, (void*)c->d_leap_resume})
     if (q) (void)hipFree(q);
   if (c->d_tf1f) (void)hipFree(c->d_tf1f);
-  if (c->d_tf1next) (void)hipFree(c->d_tf1next);
   if (c->d_tf2cols) (void)hipFree(c->d_tf2cols);
   if (c->d_list) (void)hipFree(c->d_list);
   if (c->d_views) (void)hipFree(c->d_views);
@@ -821,20 +820,22 @@ int tvk_set_tf1d(tvk_ctx* c, const uint8_t* rgba8, int n) {
   c->tf1d_n = n;
   c->tfst_dirty = true;
   int rc = ensure(c, &c->d_tf1d, &c->tf1d_cap, 4 * (size_t)n);
-  if (!rc) rc = ensure(c, &c->d_tf1f, &c->tf1f_cap, (size_t)n);
-  if (!rc) rc = ensure(c, &c->d_tf1next, &c->tf1next_cap, (size_t)n);
+  const size_t more = ((size_t)n * sizeof(uint16_t) + sizeof(float4) - 1) / sizeof(float4);
+  if (!rc) rc = ensure(c, &c->d_tf1f, &c->tf1f_cap, (size_t)n + more);
   if (rc) return rc;
-  std::vector<uint16_t> next((size_t)n);
-  for (int i = n - 1; i >= 0; --i)
-    next[(size_t)i] = rgba8[4 * (size_t)i + 3] ? (uint16_t)i : (i + 1 < n ? next[(size_t)i + 1] : (uint16_t)0xffff);
-  c->tf1d_first = std::min((int)next[0], n);
+  // texture1D of the RGBA8 table returns byte/255 (GL_NEAREST): expand once; behind
+  // it, per entry, the first one from it on with a non-zero alpha (0xffff: none)
+  std::vector<float4> f = unorm_table(rgba8, (size_t)n, more);
+  uint16_t* const next = reinterpret_cast<uint16_t*>(f.data() + n);
+  uint16_t first = 0xffffu;
   c->tf1d_clear = false;
-  for (int i = 0; i < n; ++i) c->tf1d_clear = c->tf1d_clear || rgba8[4 * (size_t)i + 3] == 0;
-  // texture1D of the RGBA8 table returns byte/255 (GL_NEAREST): expand once
-  const std::vector<float4> f = unorm_table(rgba8, (size_t)n);
+  for (int i = n - 1; i >= 0; --i) {
+    if (rgba8[4 * (size_t)i + 3]) first = (uint16_t)i; else c->tf1d_clear = true;
+    next[i] = first;
+  }
+  c->tf1d_first = std::min((int)first, n);
   HIPCHK(c, hipMemcpyAsync(c->d_tf1d, c->tf1d.data(), 4 * (size_t)n, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(c->d_tf1f, f.data(), f.size() * sizeof(float4), hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_tf1next, next.data(), next.size() * sizeof(uint16_t), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return TVK_OK;
 }
@@ -1293,7 +1294,7 @@ void fill_shade(const tvk_ctx* c, ShadeConst& S) {
   S.tf1 = c->d_tf1f;
   S.tf2f = c->d_tf2f;
   S.tf2_cols = c->d_tf2cols;
-  S.tf1_next = c->d_tf1next;
+  S.tf1_next = c->d_tf1f ? (const uint16_t*)(c->d_tf1f + c->tf1d_n) : nullptr;
   S.tf_n = c->tf1d_n;
   S.tf1_first = c->tf1d_first;
   S.tf_w = c->tf2d_w;

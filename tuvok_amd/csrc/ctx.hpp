@@ -156,12 +156,11 @@ struct tvk_ctx {
   bool tf1d_clear = false;     // the 1D TF has a transparent entry
   uint8_t* d_tf1d = nullptr;
   uint8_t* d_tf2d = nullptr;
-  float4* d_tf1f = nullptr;    // tables as the sampler returns them (byte / 255)
+  float4* d_tf1f = nullptr;    // tables as the sampler returns them (byte / 255); behind the 1D one ShadeConst::tf1_next
   float4* d_tf2f = nullptr;
   float build_ms = 0.0f;         // device time of the last bricking (build_pool)
   uint64_t* d_tf2cols = nullptr;  // 64 words: value columns of the 2D TF with a non-zero alpha
-  uint16_t* d_tf1next = nullptr;  // per 1D TF entry: the first one from it on with a non-zero alpha
-  size_t tf1d_cap = 0, tf2d_cap = 0, tf1f_cap = 0, tf2f_cap = 0, tf1next_cap = 0;
+  size_t tf1d_cap = 0, tf2d_cap = 0, tf1f_cap = 0, tf2f_cap = 0;
   // view + parameters
   ViewState V;
   bool has_view = false;
