@@ -117,6 +117,11 @@ int tvk_create(tvk_ctx** out, int device);
 void tvk_destroy(tvk_ctx* ctx);
 const char* tvk_last_error(const tvk_ctx* ctx);
 int tvk_default_params(tvk_params* p);   /* AbstrRenderer constructor defaults */
+/* Device memory that replaced or freed datasets leave behind is kept for the next
+ * one of about its size (at most 1/16 of the device's memory) until an allocation of
+ * this library fails or the device's last context is destroyed.  This call gives it
+ * back at once, for another allocator of the process; datasets that are in use stay. */
+int tvk_release_memory(int device);
 
 /* ---- dataset ------------------------------------------------------------ */
 /* Brick a linear volume (x fastest) into the ExtendedOctree layout in HBM:

@@ -105,7 +105,26 @@ static int spare_block() {
   return 0;
 }
 
+// What is kept goes when asked for; blocks in use stay.
+static int release() {
+  device_hold(0);
+  {
+    std::shared_ptr<void> a, b;
+    CHECK(device_block(&a, 20 * MB) == hipSuccess && device_block(&b, 30 * MB) == hipSuccess);
+    device_idle(a);
+    a.reset();
+    CHECK(used == 50 * MB);
+    device_release(0);
+    CHECK(used == 30 * MB);
+  }
+  CHECK(used == 30 * MB);
+  device_drop(0);
+  CHECK(used == 0);
+  return 0;
+}
+
 int main() {
+  if (release()) return 1;
   if (spare_block()) return 1;
   if (two_threads_out_of_memory()) return 1;
   std::printf("ok\n");

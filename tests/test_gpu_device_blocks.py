@@ -1,11 +1,12 @@
 """Bricking in memory that earlier datasets used: loads of several sizes in turn,
 from two threads with a renderer each, give the bricks that a first load gives."""
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
 
-from tuvok_amd import HIPRaycaster
+from tuvok_amd import HIPRaycaster, TvkError, _abi, release_memory
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +38,25 @@ def test_blocks_of_earlier_datasets():
     for t in ts:
         t.join()
     assert not bad
+
+
+def test_released_memory_is_the_device_s_again():
+    """What a replaced dataset leaves is kept, and given back when asked for."""
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert _abi.load().hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    with HIPRaycaster(0) as r:
+        release_memory()
+        r.LoadVolume(np.zeros((8, 8, 8), np.uint8), (18,) * 3, 1, max_lods=1)
+        before = free()
+        r.LoadVolume(np.zeros((400, 400, 400), np.uint8), (66,) * 3, 1, max_lods=1)
+        pool = r.GetDatasetDesc().pool_bytes
+        r.LoadVolume(np.zeros((8, 8, 8), np.uint8), (18,) * 3, 1, max_lods=1)
+        assert before - free() >= pool   # kept
+        release_memory()
+        assert before - free() <= 8 << 20
+        with pytest.raises(TvkError):
+            release_memory(-1)
+        assert r.GetBrick(0).max() == 0   # the dataset in use stays

@@ -28,7 +28,7 @@ EXPORTS = [
     "tvk_stepnet_grad", "tvk_stepnet_train", "tvk_set_step_proposal", "tvk_generate_segments",
     "tvk_batch_set_step_proposal", "tvk_leap_set_resident", "tvk_leap_render", "tvk_leap_missing",
     "tvk_leap_page_in", "tvk_leap_resume_state",
-    "tvk_set_bricks", "tvk_upload_brick", "tvk_set_pool_budget", "tvk_get_pool_stats",
+    "tvk_set_bricks", "tvk_upload_brick", "tvk_release_memory", "tvk_set_pool_budget", "tvk_get_pool_stats",
     "tvk_leap_set_request_table", "tvk_leap_requests", "tvk_pool_resident",
     "tvk_rasterize_tf2d", "tvk_set_tf2d_swatches", "tvk_set_clip_plane", "tvk_crop_dataset", "tvk_pick", "tvk_set_compat", "tvk_set_lod_filter", "tvk_set_dispatch_order", "tvk_open_uvf", "tvk_touched_mask",
 ]
@@ -198,6 +198,7 @@ def load(path=LIB_PATH):
                                      C.c_uint64]),
         "tvk_upload_brick": (C.c_int, [vp, C.c_uint32, C.c_uint64, vp, C.c_size_t]),
         "tvk_set_pool_budget": (C.c_int, [vp, C.c_uint64]),
+        "tvk_release_memory": (C.c_int, [C.c_int]),
         "tvk_leap_set_request_table": (C.c_int, [vp, C.c_uint32, C.c_uint32]),
         "tvk_leap_requests": (C.c_int, [vp, u32p, C.c_size_t, C.POINTER(C.c_size_t)]),
         "tvk_pool_resident": (C.c_int, [vp, C.POINTER(C.c_uint8), C.c_size_t]),

@@ -356,6 +356,14 @@ void tvk_destroy(tvk_ctx* c) {
   device_drop(device);
 }
 
+int tvk_release_memory(int device) {
+  int n = 0;
+  if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) return TVK_ERR_HIP;
+  if (device < 0 || device >= n) return TVK_ERR_ARG;
+  device_release(device);
+  return TVK_OK;
+}
+
 const char* tvk_last_error(const tvk_ctx* c) { return c ? c->err.c_str() : "null context"; }
 
 int tvk_load_volume(tvk_ctx* c, const void* host, int dtype, const uint64_t dims[3], const uint32_t brick[3],

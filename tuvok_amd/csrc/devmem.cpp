@@ -148,6 +148,11 @@ void device_hold(int device) {
   }
 }
 
+void device_release(int device) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  (void)trim(kept()[device]);
+}
+
 void device_drop(int device) {
   std::lock_guard<std::mutex> lk(g_mu);
   Kept& k = kept()[device];

@@ -33,6 +33,15 @@ def rotation_y(angle):
     return m
 
 
+def release_memory(device=0):
+    """Give back the device memory that replaced or freed datasets left behind (kept
+    for the next dataset of about its size otherwise): for another allocator of the
+    process, torch's for instance."""
+    rc = _abi.load().tvk_release_memory(int(device))
+    if rc != 0:
+        raise TvkError(rc, "tvk_release_memory failed")
+
+
 class HIPRaycaster:
     def __init__(self, device=0, use_only_power_of_two=False, downsample_to_8bits=False, disable_border=None):
         """AbstrRenderer(pMasterController, bUseOnlyPowerOfTwo, bDownSampleTo8Bits,
