@@ -19,25 +19,29 @@ def test_blocks_of_earlier_datasets():
         with HIPRaycaster(0) as r:
             r.LoadVolume(v, (18, 18, 18), 1)
             want.append((r.GetPool(), r.MaxGradientMagnitude()))
-    bad = []
+    bad, done = [], [0, 0]
 
     def work(start):
-        with HIPRaycaster(0) as r:
-            for k in range(8):
-                i = (start + k) % len(vols)
-                r.LoadVolume(vols[i], (18, 18, 18), 1, keep_linear=True)
-                if k % 2:
-                    r.Rebrick((34, 34, 34), 1)
-                    r.Rebrick((18, 18, 18), 1)
-                if not np.array_equal(r.GetPool(), want[i][0]) or r.MaxGradientMagnitude() != want[i][1]:
-                    bad.append((start, k))
+        try:
+            with HIPRaycaster(0) as r:
+                for k in range(8):
+                    i = (start + k) % len(vols)
+                    r.LoadVolume(vols[i], (18, 18, 18), 1, keep_linear=True)
+                    if k % 2:
+                        r.Rebrick((34, 34, 34), 1)
+                        r.Rebrick((18, 18, 18), 1)
+                    if not np.array_equal(r.GetPool(), want[i][0]) or r.MaxGradientMagnitude() != want[i][1]:
+                        bad.append((start, k))
+                    done[start] += 1
+        except Exception as e:
+            bad.append((start, e))
 
     ts = [threading.Thread(target=work, args=(s,)) for s in (0, 1)]
     for t in ts:
         t.start()
     for t in ts:
         t.join()
-    assert not bad
+    assert not bad and done == [8, 8]
 
 
 def test_released_memory_is_the_device_s_again():

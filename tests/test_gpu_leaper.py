@@ -56,6 +56,7 @@ def check_pass(r, ds, p, eye, first, resident, resume_in, rot=None):
     assert np.array_equal(miss, rmiss)
     assert mx <= 1.0 / 255 and mean < 1e-3
     assert np.abs(res - rres).max() <= 1e-4
+    assert st.unfinished == np.count_nonzero(res[..., 3] != 1000.0)   # counted by the pass
     return img, res, miss
 
 
@@ -117,6 +118,21 @@ def test_distant_view_uses_coarser_levels():
     img3, st3 = r.LeapRender(first=True)
     print(f"  samples far {far_samples} near {st3.samples}", flush=True)
     assert far_samples < st3.samples
+    r.close()
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (9, 7), (61, 43), (130, 9)])
+def test_ragged_frames_match_oracle(w, h):
+    """Fewer tiles than queues, partial tiles, queues of unequal length: every pixel
+    is passed once, first with nothing but the coarsest level resident."""
+    r, ds, p, eye = setup("fbm", w=w, h=h)
+    n = r.GetDatasetDesc().brick_count
+    resident = np.zeros(n, np.uint8)
+    resident[-1] = 1
+    r.LeapSetResident(resident)
+    img, res, miss = check_pass(r, ds, p, eye, True, resident, None)
+    r.LeapSetResident(None)
+    check_pass(r, ds, p, eye, False, None, res)
     r.close()
 
 
