@@ -93,9 +93,10 @@ def hbm_roofline(alg_bytes, ms):
 
 
 def batch_bytes(requests):
-    """V_eff of a batch, deduplicated per dataset: the union of the bricks each
-    request's counted render samples (stored bytes), plus 16 B of output and
-    4 B of descriptors per pixel.  requests: (renderer, dataset owner key,
+    """V_eff of a batch, deduplicated per dataset: the union of the bricks that
+    each request's rays march into (stored bytes, also where a ray goes by steps
+    that cannot contribute: an upper bound of what is read then), plus 16 B of
+    output and 4 B of descriptors per pixel.  requests: (renderer, dataset owner key,
     pixels); every renderer has just run a counted render."""
     union, sizes, px = {}, {}, 0
     for r, key, pixels in requests:

@@ -107,7 +107,10 @@ typedef struct {
 } tvk_dataset_desc;
 
 typedef struct {
-  uint64_t samples;      /* composited samples executed (when counting is on)   */
+  uint64_t samples;      /* samples of the march (when counting is on): every step
+                            up to the end of the ray, those gone by because they
+                            cannot contribute (1D and isosurface) included; the
+                            learned step's skipped chunks are not counted         */
   uint32_t bricks_in_list, bricks_nonempty;
   float ms;              /* device time of the last tvk_render call             */
 } tvk_stats;
@@ -361,13 +364,14 @@ int tvk_render_views(tvk_ctx* ctx, int n, const float* rots, float* host_out, tv
 /* Enable/disable the per-frame sample counter and touched-brick record (off by
  * default: costs an atomic per wave). */
 int tvk_set_count_samples(tvk_ctx* ctx, int on);
-/* Stored bytes (and count) of the bricks in which the last counted render took at
- * least one sample: summed over its views, and over the union of its views (each
- * brick once). */
+/* Stored bytes (and count) of the bricks that the rays of the last counted render
+ * marched into: summed over its views, and over the union of its views (each brick
+ * once).  A ray has at least one step in such a brick; where its steps cannot
+ * contribute they may be gone by unread. */
 int tvk_touched_bytes(tvk_ctx* ctx, uint64_t* bytes, uint64_t* bricks, uint64_t* unique_bytes,
                       uint64_t* unique_bricks);
-/* Per TOC brick: 1 where the last counted render (any of its views) took a
- * sample in the brick (V_eff, the bricks a batch's requests deduplicate). */
+/* Per TOC brick: 1 where a ray of the last counted render (any of its views)
+ * marched into the brick (V_eff, the bricks a batch's requests deduplicate). */
 int tvk_touched_mask(tvk_ctx* ctx, uint8_t* mask, size_t n);
 /* Allocation-free variant of tvk_render_views.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory while they

@@ -48,3 +48,22 @@ def test_traversal_keeps_two_waves(kernels):
     assert len(leap) == 10
     for k, (regs, spill) in leap.items():
         assert regs <= 256 and spill == 0, (k, regs, spill)
+
+
+@pytest.mark.skipif(not (os.path.exists(READELF) and os.path.exists(_abi.LIB_PATH)), reason="needs the built library")
+@pytest.mark.parametrize("pattern,count,regs,spill", [
+    (r"march_kernel<1, \w+, unsigned \w+, false, 0>", 4, 128, 0),    # 2D
+    (r"march_kernel<1, \w+, unsigned \w+, true, 0>", 4, 128, 4),
+    (r"march_kernel<2, false, unsigned \w+, \w+, 0>", 4, 128, 8),    # isosurface
+    (r"march_kernel<0, false, unsigned \w+, \w+, 0>", 4, 128, 0),    # 1D unlit, lit
+    (r"march_kernel<0, true, unsigned \w+, \w+, 0>", 4, 168, 0),
+    (r"march_kernel_learn<", 16, 168, 16),
+    (r"batch_kernel<\d, \w+, unsigned \w+, \w+, 0>", 20, 128, 2),
+    (r"batch_kernel<\d, \w+, unsigned \w+, \w+, 1>", 16, 168, 16)])
+def test_march_budgets(kernels, pattern, count, regs, spill):
+    """4 waves where 128 registers are named, 3 where 168 are, and the spills that the
+    comments beside the kernels state."""
+    found = {k: v for k, v in kernels.items() if re.match(pattern, k)}
+    assert len(found) == count
+    for k, v in found.items():
+        assert v[0] <= regs and v[1] <= spill, (k, v)

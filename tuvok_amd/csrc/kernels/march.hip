@@ -623,8 +623,9 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
       const float te = fmaxf(tn, 1.0f);  // near-plane entry when the front face is clipped
       const bool active = !done && ok && tf > te && !(MODE == 2 && eps > 0.0f && te > best_t * (1.0f + 0x1p-8f));
       if (COUNT && touched) {
-        // every ray that reaches a brick takes at least one sample there (the
-        // record is optional: the allocation-free render counts samples only)
+        // every ray that reaches a brick has at least one step there, marched or
+        // gone by (the record is optional: the allocation-free render counts
+        // samples only)
         if (__ballot(active) != 0 && lane == __builtin_amdgcn_readfirstlane(lane)) touched[fb->toc] = 1u;
       }
       if (LEARN == 0 && !active) continue;
@@ -964,8 +965,8 @@ __device__ __forceinline__ void march_tile(const ShadeConst& S, const float4* __
           // ISO_BATCH samples' loads in flight together (positions accumulated
           // one increment at a time, as step() advances them: x * 2^k is exact),
           // then composited in order; values past a termination are not used.
-          // Eight at a time measured slower on the 48-request batch (69.7
-          // against 61.7 ms: 167 against 110 VGPRs, the same 3 waves).
+          // Eight at a time measured slower on the 48-request batch, before the
+          // skipping (69.7 against 61.7 ms: 167 against 110 VGPRs).
           const V3 inc = mk(incTex.x * mlt, incTex.y * mlt, incTex.z * mlt);
           for (int i = 0; i < nsamp;) {
             int end = nsamp;
@@ -1344,9 +1345,14 @@ __device__ __forceinline__ void march_group(const MarchArgs& A) {
   });
 }
 
-// The fixed-step 2D and isosurface variants fit 128 VGPRs, 4 waves per SIMD,
-// without a spill; asked for, since the scheduler otherwise takes up to 151
-// (3 waves: 59.4 against 52.6 ms for 16 lit 2D 1080p frames of 1024^3).
+// The fixed-step 2D and isosurface variants are asked to fit 128 VGPRs, 4 waves per
+// SIMD; by itself the scheduler takes up to 151 and 3 waves.  2D without a spill (the
+// counting lit one spills 4): 52.6 against 59.4 ms for 16 lit 2D 1080p frames of
+// 1024^3.  The isosurface spills 7 or 8 outside its search loop and is faster all the
+// same: two 1080p frames of 512^3 fBm 1.20 against 1.28 ms (uint8; 3 waves: 137
+// VGPRs, no spill) and 1.26 against 1.36 (uint16), without a grid 3.03 against 3.20
+// and 3.40 against 3.62, a 2048^3 distance field 3.37 against 3.51.  The lit 1D ones
+// take 145 and 3 waves; at 4 (2 spilled) they lost 2 to 8 %.
 template <int MODE, bool LIT, typename T, bool COUNT, int LEARN>
 __global__ __launch_bounds__(256, (LEARN == 0 && MODE != 0) ? 4 : 1) void march_kernel(MarchArgs A) {
   march_group<MODE, LIT, T, COUNT, LEARN>(A);

@@ -564,14 +564,14 @@ class HIPRaycaster:
         return out
 
     def TouchedBytes(self, unique=False):
-        """Stored bytes and count of the bricks the last counted render sampled:
+        """Stored bytes and count of the bricks the last counted render marched into:
         summed over its views, or (unique=True) over their union."""
         b, n, ub, un = C.c_uint64(), C.c_uint64(), C.c_uint64(), C.c_uint64()
         self._chk(self._L.tvk_touched_bytes(self._h, C.byref(b), C.byref(n), C.byref(ub), C.byref(un)))
         return (ub.value, un.value) if unique else (b.value, n.value)
 
     def TouchedMask(self):
-        """Per TOC brick: 1 where the last counted render took a sample."""
+        """Per TOC brick: 1 where a ray of the last counted render marched into it."""
         n = self.GetDatasetDesc().brick_count
         m = np.zeros(n, np.uint8)
         self._chk(self._L.tvk_touched_mask(self._h, m.ctypes.data_as(C.POINTER(C.c_uint8)), n))
