@@ -45,9 +45,11 @@ def kernels(tmp_path_factory):
 @pytest.mark.skipif(not (os.path.exists(READELF) and os.path.exists(_abi.LIB_PATH)), reason="needs the built library")
 def test_traversal_keeps_two_waves(kernels):
     leap = {k: v for k, v in kernels.items() if k.startswith("leap_kernel<")}
-    assert len(leap) == 10
+    assert len(leap) == 12
     for k, (regs, spill) in leap.items():
-        assert regs <= 256 and spill == 0, (k, regs, spill)
+        # the form for frames of few tiles, which do not fill two waves, may take more
+        few = k == "leap_kernel<0, true, unsigned short, true>"
+        assert regs <= (264 if few else 256) and spill == 0, (k, regs, spill)
 
 
 @pytest.mark.skipif(not (os.path.exists(READELF) and os.path.exists(_abi.LIB_PATH)), reason="needs the built library")

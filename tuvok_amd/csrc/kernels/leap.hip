@@ -290,8 +290,9 @@ __device__ __forceinline__ uint32_t compute_lod(const LeapArgs& A, float depth) 
   return min((uint32_t)(A.nlod - 1), lod);
 }
 
-// cols: the 2D TF's column mask (64 words, MODE 1) in LDS
-template <int MODE, bool LIT, typename T>
+// cols: the 2D TF's column mask (64 words, MODE 1) in LDS.  RANGE: the steps whose
+// cross loads apply are found per segment; without it by one ballot per step.
+template <int MODE, bool LIT, typename T, bool RANGE>
 __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int lane, const uint64_t* cols) {
   const int tx = (int)(tile % A.tiles_x), ty = (int)(tile / A.tiles_x);
   const int px = tx * 8 + (lane & 7), py = ty * 8 + (lane >> 3);
@@ -449,12 +450,45 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
             const V3 q = p - tr;
             return mk(quotient(q.x, sc.x, rsc.x), quotient(q.y, sc.y, rsc.y), quotient(q.z, sc.z, rsc.z));
           };
-          for (int i = 0; i < steps; ++i) {
+          // The steps whose 4x4x4 neighbourhood lies inside the brick, one range
+          // per segment (the raycaster's rule and margin: each addition of a
+          // position below n rounds by at most n 2^-24, so after i < steps of
+          // them the drift is below steps n 2^-24 voxels).  Every lane takes its
+          // steps before the range, in it and after it as three loops, so only
+          // the few steps next to a brick face pay for per-tap gathers; decided
+          // by one ballot per step, a wave gathered whenever any of its 64 rays
+          // was next to a face.
+          int in_lo = 0, in_hi = -1;
+          if constexpr (RANGE) {
+            float lo = 0.0f, hi = (float)(steps - 1);
+            const float pc[3] = {pin.x, pin.y, pin.z}, sp[3] = {step.x, step.y, step.z};
+            const int nn3[3] = {nx, ny, nz};
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+              const float na = (float)nn3[a], u0 = pc[a] - 0.5f, du = sp[a];
+              const float margin = 0.0625f + (float)steps * na * 0x1p-23f;
+              const float ulo = 1.0f + margin, uhi = na - 2.0f - margin;   // floor(u) in [1, n - 3]
+              if (!(ulo <= uhi) || !(fabsf(u0) < 0x1p24f) || !(fabsf(du) < 0x1p24f)) {
+                hi = -1.0f;
+              } else if (du == 0.0f) {
+                if (!(u0 >= ulo && u0 <= uhi)) hi = -1.0f;
+              } else {
+                const float t1 = (ulo - u0) / du, t2 = (uhi - u0) / du;
+                lo = fmaxf(lo, fminf(t1, t2));
+                hi = fminf(hi, fmaxf(t1, t2));
+              }
+            }
+            if (hi >= lo) { in_lo = (int)ceilf(lo); in_hi = (int)floorf(hi); }
+          }
+          int i = 0;
+          for (int part = 0; part < (RANGE ? 3 : 1) && !done; ++part) {
+          const int end = !RANGE ? steps : part == 0 ? (in_hi >= in_lo ? min(in_lo, steps) : steps) : (part == 1 ? min(in_hi + 1, steps) : steps);
+          for (; i < end; ++i) {
             ++ns;
             // value (and, for gradients, the cross) from the 32-voxel cross when
             // every active lane's neighbourhood lies inside its brick
             LeapCross<T> X;
-            const bool cross = MODE != 2 && (LIT || MODE == 1) && __ballot(!X.coords(nx, ny, nz, b)) == 0;
+            const bool cross = MODE != 2 && (LIT || MODE == 1) && (!RANGE || part == 1) && __ballot(!X.coords(nx, ny, nz, b)) == 0;
             const float data = cross ? X.value(bd, nx, ny) : sample_vox_fast<T>(bd, nx, ny, nz, b);
             auto grad = [&]() { return cross ? X.gradient() : gradient_vox<T>(bd, nx, ny, nz, b); };
             if constexpr (MODE == 2) {
@@ -519,6 +553,7 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
             if (acc[3] > 0.99f) { done = true; break; }
             b = b + step;
           }
+          }
           if (!done) cur = (b - tr) / sc;
         } else {
           cur = bexit + direction * voxelSize / rayLength;
@@ -570,14 +605,10 @@ __device__ __forceinline__ void leap_tile(const LeapArgs& A, uint32_t tile, int 
 }
 
 // persistent grid: every wave pulls 8x8 tiles from its XCD's queue, then from the
-// others' (pull_tiles).  XCD x has the tiles x, x + 8, ...: every queue then holds
-// its share of the long rays in the frame's middle, and the short ones below it
-// come last in all of them (1080p over 512^3 with every level, kernel, against a
-// band of rows per XCD: unlit 1D 0.94 -> 0.83 ms uint8 and 0.99 -> 0.86 uint16,
-// lit 2D 4.39 -> 4.13 and 4.65 -> 4.31, isosurface 1.36 -> 1.26 and 1.41 -> 1.27).
-// No cap of waves: asked for 2 per SIMD the scheduler waits for loads one by one
-// (lit 1D uint8: 2.87 -> 3.64 ms).
-template <int MODE, bool LIT, typename T>
+// others' (pull_tiles; launch_leap says which tiles an XCD has).  No cap of waves:
+// asked for 2 per SIMD the scheduler waits for loads one by one (lit 1D uint8, 1080p
+// over 512^3: 2.87 -> 3.64 ms).
+template <int MODE, bool LIT, typename T, bool RANGE>
 __global__ __launch_bounds__(256) void leap_kernel(LeapArgs A) {
   __shared__ uint64_t s_cols[MODE == 1 ? 64 : 1];
   const int lane = threadIdx.x & 63;
@@ -586,10 +617,10 @@ __global__ __launch_bounds__(256) void leap_kernel(LeapArgs A) {
     __syncthreads();   // the only workgroup barrier
   }
   pull_tiles(A.queues, A.xcd_items,
-             [&](uint32_t x, uint32_t t) { leap_tile<MODE, LIT, T>(A, t * 8u + x, lane, s_cols); });
+             [&](uint32_t x, uint32_t t) { leap_tile<MODE, LIT, T, RANGE>(A, x * A.tile_x + t * A.tile_t, lane, s_cols); });
 }
 
-template <int M, bool L, typename T>
+template <int M, bool L, typename T, bool RANGE>
 void launch_leap_one(const LeapArgs& a, uint32_t blocks, hipStream_t st) {
   // the workgroups the device holds at once, no more than the tiles keep busy,
   // a multiple of 8
@@ -597,27 +628,60 @@ void launch_leap_one(const LeapArgs& a, uint32_t blocks, hipStream_t st) {
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(leap_kernel<M, L, T>), 256,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(leap_kernel<M, L, T, RANGE>), 256,
                                                    0) != hipSuccess || per_cu <= 0)
     per_cu = 1;
   blocks = std::min(blocks, ((uint32_t)per_cu * (uint32_t)cus + 7u) & ~7u);
-  hipLaunchKernelGGL((leap_kernel<M, L, T>), dim3(blocks), dim3(256), 0, st, a);
+  hipLaunchKernelGGL((leap_kernel<M, L, T, RANGE>), dim3(blocks), dim3(256), 0, st, a);
 }
 
 }  // namespace
 
-hipError_t launch_leap(const LeapArgs& a, int bpv, hipStream_t st) {
+// Which tiles an XCD has, and which form of the step loop runs (kernel times, 1080p
+// over 512^3 with every level unless another size is named):
+// - Tiles x, x + 8, ... on XCD x: every queue holds its share of the long rays in the
+//   frame's middle.  Against a band of rows each: unlit 1D 0.92 -> 0.82 ms uint8 and
+//   0.99 -> 0.85 uint16, lit 2D 4.40 -> 4.10 and 4.62 -> 4.22, isosurface 1.33 -> 1.25.
+//   1D frames of few tiles keep the bands, whose neighbouring rays share an L2 (whole
+//   passes: 283x513 lit over 256^3 0.77 against 0.83 ms, 797x297 unlit over 1024^3
+//   0.417 against 0.430).
+// - The step ranges (RANGE) are the 2D form: they fit 2 waves per SIMD and rays next to
+//   a brick face gather alone (771x364 over 512^3: 1.54 against 1.65 ms).  In the lit
+//   1D uint16 kernel they cost the second wave (258 registers): without them 2.62
+//   against 3.80 ms, uint8 2.55 against 3.10.  Frames of few tiles do not fill two
+//   waves and take them (283x513 over 256^3: 0.77 against 0.90 ms, 640x640 over 512^3
+//   1.41 against 1.49).
+// The line between few and many lies between 640x640 and 900x800, where both forms of
+// either rule are mostly within 3 % of each other (at most 7).
+constexpr uint32_t LEAP_FEW_TILES = 8192;
+
+hipError_t launch_leap(const LeapArgs& args, int bpv, hipStream_t st) {
+  LeapArgs a = args;
+  const bool few = a.mode == 0 && a.ntiles <= LEAP_FEW_TILES;
+  if (few) {
+    chunk_items(a.ntiles, a.xcd_items);
+    a.tile_x = a.xcd_items[0];
+    a.tile_t = 1;
+  } else {
+    for (uint32_t x = 0; x < 8; ++x) a.xcd_items[x] = (a.ntiles + 7u - x) / 8u;
+    a.tile_x = 1;
+    a.tile_t = 8;
+  }
   const uint32_t blocks = (a.xcd_items[0] + 3u) / 4u * 8u;   // four tiles a workgroup, every XCD alike
   if (blocks == 0) return hipSuccess;
   const bool u16 = bpv == 2, lit = a.lighting != 0;
   if (a.mode == 0) {
-    if (lit) { if (u16) launch_leap_one<0, true, uint16_t>(a, blocks, st); else launch_leap_one<0, true, uint8_t>(a, blocks, st); }
-    else { if (u16) launch_leap_one<0, false, uint16_t>(a, blocks, st); else launch_leap_one<0, false, uint8_t>(a, blocks, st); }
+    if (lit) {
+      if (few) { if (u16) launch_leap_one<0, true, uint16_t, true>(a, blocks, st); else launch_leap_one<0, true, uint8_t, true>(a, blocks, st); }
+      else { if (u16) launch_leap_one<0, true, uint16_t, false>(a, blocks, st); else launch_leap_one<0, true, uint8_t, false>(a, blocks, st); }
+    } else {
+      if (u16) launch_leap_one<0, false, uint16_t, false>(a, blocks, st); else launch_leap_one<0, false, uint8_t, false>(a, blocks, st);
+    }
   } else if (a.mode == 1) {
-    if (lit) { if (u16) launch_leap_one<1, true, uint16_t>(a, blocks, st); else launch_leap_one<1, true, uint8_t>(a, blocks, st); }
-    else { if (u16) launch_leap_one<1, false, uint16_t>(a, blocks, st); else launch_leap_one<1, false, uint8_t>(a, blocks, st); }
+    if (lit) { if (u16) launch_leap_one<1, true, uint16_t, true>(a, blocks, st); else launch_leap_one<1, true, uint8_t, true>(a, blocks, st); }
+    else { if (u16) launch_leap_one<1, false, uint16_t, true>(a, blocks, st); else launch_leap_one<1, false, uint8_t, true>(a, blocks, st); }
   } else if (a.mode == 2) {
-    if (u16) launch_leap_one<2, false, uint16_t>(a, blocks, st); else launch_leap_one<2, false, uint8_t>(a, blocks, st);
+    if (u16) launch_leap_one<2, false, uint16_t, false>(a, blocks, st); else launch_leap_one<2, false, uint8_t, false>(a, blocks, st);
   } else {
     return hipErrorInvalidValue;
   }

@@ -364,7 +364,6 @@ int tvk_leap_render(tvk_ctx* c, int first, float* host_out, tvk_leap_stats* st) 
     HIPCHK(c, launch_fill_u32(c->d_queues, QUEUE_WORDS + 1, 0u, c->stream));
     a.unfinished = c->d_queues + QUEUE_WORDS;
     a.queues = c->d_queues;
-    for (uint32_t x = 0; x < 8; ++x) a.xcd_items[x] = (a.ntiles + 7u - x) / 8u;   // tiles x, x + 8, ...
   }
   if (c->count) HIPCHK(c, hipMemsetAsync(c->d_counter, 0, sizeof(unsigned long long), c->stream));
   HIPCHK(c, hipEventRecord(c->ev[6], c->stream));

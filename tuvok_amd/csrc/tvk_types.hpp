@@ -242,10 +242,11 @@ struct LeapArgs {
   int nlod, W, H, first, lighting, mode, overlap;
   uint32_t tiles_x;
   // QUEUE_WORDS words cleared before the launch: the grid is persistent and its
-  // waves pull tiles 0 .. ntiles-1, tile t from the queue of XCD t mod 8
+  // waves pull tiles 0 .. ntiles-1 from 8 queues, one per XCD
   unsigned int* queues;
   uint32_t ntiles;
-  uint32_t xcd_items[8];        // tiles of each XCD's queue
+  uint32_t xcd_items[8];        // tiles of each XCD's queue: item i of XCD x is tile x tile_x + i tile_t
+  uint32_t tile_x, tile_t;
 };
 
 // the 8 contiguous chunks of a persistent launch's n tiles
