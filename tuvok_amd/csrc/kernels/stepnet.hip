@@ -272,7 +272,7 @@ __global__ __launch_bounds__(64) void sn_reduce(const float* __restrict__ part, 
 // packed again, and the batch's loss at loss[0].  A step was four launches and a
 // 4-byte download the host waited for; with the losses kept on the device until
 // the epoch's end it is two launches and no wait (100000 samples, 2 epochs of
-// 25 batches: 3.44 -> 1.5 ms).  One wave per workgroup spreads the 6466 chains
+// 25 batches: 3.45 -> 1.78 ms).  One wave per workgroup spreads the 6466 chains
 // over the CUs.
 __global__ __launch_bounds__(64) void sn_step(const float* __restrict__ part, int tiles, float* __restrict__ th,
                                               float* __restrict__ m, float* __restrict__ v, float lr, float b1,
